@@ -1,18 +1,19 @@
-// K1: paged verify attention for gfx950 (MFMA 16x16x32 bf16).
+// K1: paged verify attention for gfx950 (MFMA 16x16x32 bf16; prefill
+// 32x32x16).
 //
-// Unit of work: one wave (64 threads) runs a *segment* -- one query tile of
+// Unit of work: one wave (64 threads) runs a *segment* -- the query tile of
 // one sequence against a contiguous key range, for one kv head.  A query
-// tile is up to 64/G consecutive query positions of a sequence times the G
-// query heads that share the kv head (G = Hq / Hkv), padded to NT*16 columns
-// (NT = 1, 2, 4); a verify step (k+1 positions) is a single tile, a prefill
-// is many.  Each tile only walks the keys its last row can see.  Segments
+// tile is up to 64/G query positions of a sequence times the G query heads
+// that share the kv head (G = Hq / Hkv), padded to NT*16 columns (NT = 1, 2,
+// 4): every row of a verify step (k+1 positions).  Sequences with more rows
+// than one such tile (prefill) run on the wide-tile kernel below.  Segments
 // come from one of two decompositions:
 //   * stream (single-tile sequences of at most 32 rows over an FP8 cache):
 //     per kv head the key chunks of all sequences are laid end to end and
 //     cut into one equal range per SIMD of the device, so every wave streams
 //     the same number of keys whatever the length mix;
-//   * fixed (everything else): one workgroup per (kv head, sequence, query
-//     tile, key split).  For bf16 tiles of up to 32 rows eight waves share a
+//   * fixed (everything else): one workgroup per (kv head, sequence, key
+//     split).  For bf16 tiles of up to 32 rows eight waves share a
 //     2816-key split (wave w takes chunks w, w+8, ...) and fold their
 //     softmax states together in LDS; for single-tile 17-32-row tiles whose
 //     segments fill every CU once or twice, four waves share a whole
@@ -108,7 +109,7 @@ struct AttnParams {
   float* ws_o;
   float* ws_lse;
   int32_t split_len, max_splits;
-  int32_t qtile, n_qtiles;                            // query positions per workgroup
+  int32_t qtile, n_qtiles;                            // query positions per tile (wide-tile kernel: several)
   // stream decomposition (one query tile per sequence)
   int32_t min_range_chunks, max_range_chunks;
   int32_t* row_nsplit;                                // [num_tokens] split count per query row
@@ -284,10 +285,10 @@ constexpr bool k_staged(bool fp8, bool pipe, int wps) {
   return NVA_K_STAGE && (fp8 || (!pipe && wps > 1));
 }
 
-// One segment of work: the query tile qt of sequence seq (all its rows
+// One segment of work: the query tile of sequence seq (all its rows
 // for kv head kvh; the sequence's rows start at q_start, it has q_len query
 // rows and L keys) against keys [kv_begin, kv_end), which is split `split`
-// of the `nsplit` splits covering the keys the tile can see.  lane_blk is
+// of the `nsplit` splits covering its keys.  lane_blk is
 // split_block_ids(p, seq, kv_begin).  A single split
 // writes the bf16 output; otherwise a normalised fp32 partial and its
 // log-sum-exp go to the workspace for combine_kernel.
@@ -297,11 +298,10 @@ constexpr bool k_staged(bool fp8, bool pipe, int wps) {
 // wave 0 writes the result.  `vst` then holds WPS stages.
 template <int NT, bool FP8, bool PIPE, int WPS>
 __device__ __forceinline__ void attend_segment(const AttnParams& p, uint32_t* vst, bf16x8_t* qst,
-                                               const int kvh, const int seq, const int qt,
-                                               const int q_start, const int q_len, const int L,
-                                               const int kv_begin, const int kv_end,
-                                               const int split, const int nsplit,
-                                               const int lane_blk) {
+                                               const int kvh, const int seq, const int q_start,
+                                               const int q_len, const int L, const int kv_begin,
+                                               const int kv_end, const int split,
+                                               const int nsplit, const int lane_blk) {
   static_assert(WPS == 1 || !PIPE, "shared segments use the single-buffer loop");
   static_assert(WPS == 1 || (NT <= 2 && (8 * kWave * 4 + 2 * kWave) <= kVStage),
                 "a wave's parked state must fit one V stage per column tile");
@@ -313,12 +313,7 @@ __device__ __forceinline__ void attend_segment(const AttnParams& p, uint32_t* vs
   uint32_t* const stage = vst + wv * kVStage;           // this wave's V stage
   uint32_t* const kstage = KST ? vst + (WPS + wv) * kVStage : stage;  // its K stage
 
-  // this tile's query positions: j0 .. j0 + jn - 1 of the sequence
-  const int j0 = qt * p.qtile;
-  const int jn = (q_len - j0 < p.qtile) ? q_len - j0 : p.qtile;
-  const int rows = jn * p.group;
-  // keys any row of the tile can see (bottom-right causal)
-  const int kv_limit = L - q_len + j0 + jn;
+  const int rows = q_len * p.group;
 
   float kscale = 1.0f, vscale = 1.0f;
   if (FP8) {
@@ -340,7 +335,7 @@ __device__ __forceinline__ void attend_segment(const AttnParams& p, uint32_t* vs
   for (int nt = 0; nt < NT; ++nt) {
     const int n = nt * 16 + m16;
     const int nn = n < rows ? n : 0;
-    const int j = j0 + nn / p.group, hh = nn % p.group;
+    const int j = nn / p.group, hh = nn % p.group;
     const uint16_t* qp = p.q + static_cast<int64_t>(q_start + j) * p.q_row_stride +
                          static_cast<int64_t>(kvh * p.group + hh) * p.q_head_stride;
 #pragma unroll
@@ -410,7 +405,7 @@ __device__ __forceinline__ void attend_segment(const AttnParams& p, uint32_t* vs
     const int raw = __builtin_amdgcn_readlane(lane_blk, kb / p.block_size - first_blk);
     ch.valid = raw >= 0 && raw < p.num_blocks;
     const int pblk = ch.valid ? raw : 0;
-    const int visible = kv_limit - kb < kChunk ? kv_limit - kb : kChunk;
+    const int visible = L - kb < kChunk ? L - kb : kChunk;
     const int nrec = ch.valid ? visible * static_cast<int>(tokb) : 0;
     const int64_t tile = (static_cast<int64_t>(pblk) * p.blk_stride +
                           static_cast<int64_t>(kvh) * p.head_stride +
@@ -533,7 +528,7 @@ __device__ __forceinline__ void attend_segment(const AttnParams& p, uint32_t* vs
     // sequence end) is masked, behind a uniform branch: written as a select
     // per score, the compare and select ran on every chunk (40 VALU
     // instructions of ~170 per chunk).
-    const bool full = kb + kChunk - 1 <= L - q_len + j0 && kb + kChunk <= kv_limit;
+    const bool full = kb + kChunk - 1 <= L - q_len && kb + kChunk <= L;
     if (!full) {
       const int rel = kb + 4 * g;
 #pragma unroll
@@ -708,7 +703,7 @@ __device__ __forceinline__ void attend_segment(const AttnParams& p, uint32_t* vs
       const float inv = lsum > 0.0f ? vscale / lsum : 0.0f;
       const int n = nt * 16 + m16;
       if (n < rows) {
-        const int j = j0 + n / p.group, hh = n % p.group;
+        const int j = n / p.group, hh = n % p.group;
         const int tok = q_start + j;
         const int h = kvh * p.group + hh;
         const int64_t slot = (static_cast<int64_t>(tok) * p.hq + h) * p.max_splits + split;
@@ -755,7 +750,7 @@ __device__ __forceinline__ void attend_segment(const AttnParams& p, uint32_t* vs
     const float inv = lsum > 0.0f ? vscale / lsum : 0.0f;
     const int n = nt * 16 + m16;
     if (n < rows) {
-      const int j = j0 + n / p.group, hh = n % p.group;
+      const int j = n / p.group, hh = n % p.group;
       const int tok = q_start + j;
       const int h = kvh * p.group + hh;
       const int64_t slot = (static_cast<int64_t>(tok) * p.hq + h) * p.max_splits + split;
@@ -835,10 +830,8 @@ __device__ __forceinline__ int stream_chunks(const AttnParams& p, int seq) {
   return (q_len > 0 && L > 0) ? (L + kChunk - 1) / kChunk : 0;
 }
 
-// Fixed decomposition, one wave per (kv head, sequence, query tile, split):
-// used when a sequence has several query tiles (prefill).
-// Dispatch order (x fastest): kv head, sequence, then (query tile, split)
-// slowest, so every full split is dispatched before the shorter trailing
+// Fixed decomposition, WPS waves per (kv head, sequence, split).
+// Dispatch order (x fastest): kv head, sequence, then the split slowest, so every full split is dispatched before the shorter trailing
 // splits and the empty splits that pad the grid come last.
 // Two waves per SIMD fit the register budget of tiles up to 32 columns;
 // 64-column tiles (NT = 4) need the full register file of one wave.
@@ -853,40 +846,35 @@ paged_attention_kernel(AttnParams p) {
   const int kvh = blockIdx.x;
   const int row = blockIdx.y;
   const int seq = (p.pair_rows > 0 && row >= p.pair_rows) ? p.num_seqs - 1 - (row - p.pair_rows) : row;
-  const int split = blockIdx.z % p.max_splits;
-  const int qt = blockIdx.z / p.max_splits;
+  const int split = blockIdx.z;
   const int kv_begin = split * p.split_len;
   const int lane_blk = split_block_ids(p, seq, kv_begin);
   int q_start, q_len, L, q_raw;
   seq_geometry_uniform(p, seq, q_start, q_len, L, &q_raw);
-  const int j0 = qt * p.qtile;
-  const int jn = (q_len - j0 < p.qtile) ? q_len - j0 : p.qtile;
-  const int kv_limit = L - q_len + j0 + jn;  // meaningful when jn > 0
-  const int nsplit = kv_limit > 0 ? (kv_limit + p.split_len - 1) / p.split_len : 0;
+  const int nsplit = L > 0 ? (L + p.split_len - 1) / p.split_len : 0;
   const bool note = kvh == 0 && split == 0 && p.row_nsplit;
   // rows past max_seqlen_q, if any, are cleared by one workgroup
-  const bool clip_owner = kvh == 0 && split == 0 && qt == p.n_qtiles - 1 && q_raw > q_len;
+  const bool clip_owner = kvh == 0 && split == 0 && q_raw > q_len;
   // one branch on the whole geometry, so every geometry load is issued
   // before the first wait
-  if (jn <= 0 || kv_begin >= kv_limit) {
-    if (jn > 0) {
-      if (note) note_rows(p, seq, qt, nsplit);
-      if (kv_limit <= 0 && split == 0) zero_tile(p, kvh, seq, qt);
+  if (q_len <= 0 || kv_begin >= L) {
+    if (q_len > 0) {
+      if (note) note_rows(p, seq, 0, nsplit);
+      if (L <= 0 && split == 0) zero_tile(p, kvh, seq, 0);
     }
     if (clip_owner) clear_clipped_rows(p, q_start, q_len, q_raw, threadIdx.x, blockDim.x);
     return;
   }
-  if (note) note_rows(p, seq, qt, nsplit);
-  const int kv_end = kv_begin + p.split_len < kv_limit ? kv_begin + p.split_len : kv_limit;
-  attend_segment<NT, FP8, PIPE, WPS>(p, vst, qst, kvh, seq, qt, q_start, q_len, L, kv_begin, kv_end,
+  if (note) note_rows(p, seq, 0, nsplit);
+  const int kv_end = kv_begin + p.split_len < L ? kv_begin + p.split_len : L;
+  attend_segment<NT, FP8, PIPE, WPS>(p, vst, qst, kvh, seq, q_start, q_len, L, kv_begin, kv_end,
                                      split, nsplit, lane_blk);
   if (clip_owner) clear_clipped_rows(p, q_start, q_len, q_raw, threadIdx.x, blockDim.x);
 }
 
 // ---------------------------------------------------------------- shared-tile kernel
-// Tiles of 33-64 rows (64-row verify tiles of GQA group 8 with k = 7, and the
-// prefill tiles of every geometry): WPT waves share one segment (kv head,
-// sequence, query tile, key split), wave w owning the NTW = 4 / WPT column
+// Tiles of 33-64 rows (64-row verify tiles of GQA group 8 with k = 7): WPT
+// waves share one segment (kv head, sequence, key split), wave w owning the NTW = 4 / WPT column
 // tiles 16 NTW w .. of the 64 query columns over every key of the split,
 // so each wave finishes its own columns and nothing is merged.
 //   * The workgroup loads each 32-key chunk once, cooperatively: thread t
@@ -918,35 +906,31 @@ paged_attention_tile_kernel(AttnParams p) {
 
   const int kvh = blockIdx.x;
   const int seq = blockIdx.y;
-  const int split = blockIdx.z % p.max_splits;
-  const int qt = blockIdx.z / p.max_splits;
+  const int split = blockIdx.z;
   const int kv_begin = split * p.split_len;
   const int lane_blk = split_block_ids(p, seq, kv_begin);
   int q_start, q_len, L, q_raw;
   seq_geometry_uniform(p, seq, q_start, q_len, L, &q_raw);
-  const int j0 = qt * p.qtile;
-  const int jn = (q_len - j0 < p.qtile) ? q_len - j0 : p.qtile;
-  const int kv_limit = L - q_len + j0 + jn;  // meaningful when jn > 0
-  const int nsplit = kv_limit > 0 ? (kv_limit + p.split_len - 1) / p.split_len : 0;
+  const int nsplit = L > 0 ? (L + p.split_len - 1) / p.split_len : 0;
   const bool note = kvh == 0 && split == 0 && p.row_nsplit;
-  const bool clip_owner = kvh == 0 && split == 0 && qt == p.n_qtiles - 1 && q_raw > q_len;
-  if (jn <= 0 || kv_begin >= kv_limit) {
-    if (jn > 0) {
-      if (note) note_rows(p, seq, qt, nsplit);
-      if (kv_limit <= 0 && split == 0) zero_tile(p, kvh, seq, qt);
+  const bool clip_owner = kvh == 0 && split == 0 && q_raw > q_len;
+  if (q_len <= 0 || kv_begin >= L) {
+    if (q_len > 0) {
+      if (note) note_rows(p, seq, 0, nsplit);
+      if (L <= 0 && split == 0) zero_tile(p, kvh, seq, 0);
     }
     if (clip_owner) clear_clipped_rows(p, q_start, q_len, q_raw, threadIdx.x, blockDim.x);
     return;
   }
-  if (note) note_rows(p, seq, qt, nsplit);
-  const int kv_end = kv_begin + p.split_len < kv_limit ? kv_begin + p.split_len : kv_limit;
+  if (note) note_rows(p, seq, 0, nsplit);
+  const int kv_end = kv_begin + p.split_len < L ? kv_begin + p.split_len : L;
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int g = lane >> 4;
   const int m16 = lane & 15;
-  const int rows = jn * p.group;
+  const int rows = q_len * p.group;
   const float sl2 = p.scale_log2;
 
   // ---- this wave's query operands (padding columns zero) and causal limits
@@ -956,7 +940,7 @@ paged_attention_tile_kernel(AttnParams p) {
   for (int nt = 0; nt < NTW; ++nt) {
     const int n = (wv * NTW + nt) * 16 + m16;
     const int nn = n < rows ? n : 0;
-    const int j = j0 + nn / p.group, hh = nn % p.group;
+    const int j = nn / p.group, hh = nn % p.group;
     const uint16_t* qp = p.q + static_cast<int64_t>(q_start + j) * p.q_row_stride +
                          static_cast<int64_t>(kvh * p.group + hh) * p.q_head_stride;
 #pragma unroll
@@ -989,7 +973,7 @@ paged_attention_tile_kernel(AttnParams p) {
     const int kb = kv_begin + cc * kChunk;
     const int raw = chunk_block(cc);
     const bool valid = live && raw >= 0 && raw < p.num_blocks;
-    const int visible = kv_limit - kb < kChunk ? kv_limit - kb : kChunk;
+    const int visible = L - kb < kChunk ? L - kb : kChunk;
     const int nrec = valid ? visible * static_cast<int>(tokb) : 0;
     const int64_t tile = (static_cast<int64_t>(valid ? raw : 0) * p.blk_stride +
                           static_cast<int64_t>(kvh) * p.head_stride +
@@ -1047,7 +1031,7 @@ paged_attention_tile_kernel(AttnParams p) {
         for (int kt = 0; kt < 2; ++kt) sacc[kt][nt] = mfma(kop[kt], qv[nt][s], sacc[kt][nt]);
     }
     // masked only past a causal limit, behind a uniform branch (as above)
-    const bool full = kb + kChunk - 1 <= L - q_len + j0 && kb + kChunk <= kv_limit;
+    const bool full = kb + kChunk - 1 <= L - q_len && kb + kChunk <= L;
     if (!full) {
       const int rel = kb + 4 * g;
 #pragma unroll
@@ -1153,7 +1137,7 @@ paged_attention_tile_kernel(AttnParams p) {
     const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
     const int n = (wv * NTW + nt) * 16 + m16;
     if (n < rows) {
-      const int j = j0 + n / p.group, hh = n % p.group;
+      const int j = n / p.group, hh = n % p.group;
       const int tok = q_start + j;
       const int h = kvh * p.group + hh;
       const int64_t slot = (static_cast<int64_t>(tok) * p.hq + h) * p.max_splits + split;
@@ -1177,6 +1161,388 @@ paged_attention_tile_kernel(AttnParams p) {
         }
       }
       if (nsplit > 1 && g == 0) p.ws_lse[slot] = lsum > 0.0f ? m_run[nt] + __log2f(lsum) : -INFINITY;
+    }
+  }
+  if (clip_owner) clear_clipped_rows(p, q_start, q_len, q_raw, threadIdx.x, blockDim.x);
+}
+
+// ---------------------------------------------------------------- wide-tile kernel
+// Sequences of several query tiles (every prefill): a workgroup of NW waves
+// takes 32 NW query rows (32 per wave) of one sequence and kv head over a key
+// range, 64 keys a step, on the 32x32x16 MFMA.
+//   * What bounds it: matrix cores and the softmax's vector instructions
+//     about equally (per 64 keys and wave: 32 MFMAs and ~130 VALU
+//     instructions, 32 of them exponentials), then the LDS reads, which are
+//     why a wave holds 32 columns: each K and V byte read from LDS feeds 32
+//     columns, twice the 16-column tiles' share, and each byte read from L2
+//     feeds 32 NW.
+//   * S^T = K . Q^T with keys as M: lane l = 32 h + c holds, for query column
+//     c, the keys 8 b + 4 h + i (b, i = 0..3) of each 32-key tile in
+//     accumulator element 4 b + i.  Elements 8 t .. 8 t + 7 are, in order, the
+//     k-slots of lane half h in the B operand of slice t of O^T += V^T . P^T,
+//     if slot j of half h stands for key 16 t + 8 (j / 4) + 4 h + j % 4, so P
+//     goes from accumulator to operand by rounding alone; V^T is read from
+//     LDS in that key order by two transpose loads (wide_v_operand).
+//   * K/V tiles are loaded into registers two steps ahead, staged (FP8:
+//     dequantised to bf16) into one of two LDS buffers one step ahead, with
+//     one barrier per step.  Rows of 68 dwords for K (16-byte reads of 8 rows
+//     cover all banks) and 72 for V (a 16-lane transpose load reads four rows
+//     of 32 bytes, 8 banks apart).
+//   * The heaviest query tiles (the last ones, under the causal mask) are
+//     dispatched first, and the kv head is the fastest grid dimension, so
+//     that with eight kv heads an XCD's L2 holds one head's pages.
+//   * KG = 2: two key groups of NW waves take the 64-key steps in turn, each
+//     with buffers of its own, and the second's states are folded into the
+//     first's through LDS at the end (wide_plan says when).
+// Against the 64-row tiles (which read K and V from LDS once per 16 columns
+// and from L2 once per 64 rows; FP8 ones on one wave): 16384 tokens as
+// 8192-token prompts at Qwen3-8B 2974 -> 1091 us (370 -> 1008 TFLOP/s of the
+// unmasked products; MFMAs busy 47% of the cycles), 256-2048-token prompts
+// 511 -> 314, over FP8 pages 4196 -> 1045 and 536 -> 256.  What was tried and
+// did not help: the next step's scores issued among this step's exponentials
+// (spills: 1389 us), s_setprio around the MFMAs (1117), query and output rows
+// through LDS as whole lines (+0-4%), light and heavy query tiles alternated
+// (+5%).
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+constexpr int kWideKeys = 64;
+constexpr int kWideKPitch = 68, kWideVPitch = 80;   // dwords per staged row
+constexpr int kWideBuf = kWideKeys * (kWideKPitch + kWideVPitch);
+
+__device__ __forceinline__ f32x16_t mfma32(bf16x8_t a, bf16x8_t b, f32x16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// V^T operand of head_dim tile dt (d = 32 dt + lane % 32) and key slice t
+// (16 keys) from staged rows: transpose load r (0, 1) hands lane 32 h + c the
+// keys 16 t + 8 r + 4 h .. + 3 (see v_operand_tr for the instruction).
+__device__ __forceinline__ bf16x8_t wide_v_operand(const uint32_t* rows, int lane, int t, int dt) {
+  const int h = lane >> 5, dh = (lane >> 4) & 1, i = lane & 15;
+  uint32_t* p0 = const_cast<uint32_t*>(rows) + (16 * t + 4 * h + (i >> 2)) * kWideVPitch + 16 * dt +
+                 8 * dh + 2 * (i & 3);
+  const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(p0));
+  const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(p0 + 8 * kWideVPitch));
+  return bf16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+}
+
+template <int NW, int KG, bool FP8>
+__global__ void __launch_bounds__(kWave * NW * KG, 2)
+paged_attention_wide_kernel(AttnParams p) {
+  constexpr int kThreads = kWave * NW;                   // of one key group
+  constexpr int kEsz = FP8 ? 1 : 2;
+  constexpr int kRowGran = kD * kEsz / 16;               // 16-byte granules per K or V row
+  constexpr int kPer = kWideKeys * kRowGran / kThreads;  // a thread's granules of K (and of V)
+  static_assert(kPer >= 1, "every thread loads at least one granule");
+  static_assert(KG == 1 || NW * kWave * (64 + 2) <= 2 * kWideBuf * KG, "parked states fit");
+  __shared__ __attribute__((aligned(16))) uint32_t lds[2 * kWideBuf * KG];
+
+  const int kvh = blockIdx.x;
+  const int seq = blockIdx.y;
+  const int split = blockIdx.z % p.max_splits;
+  const int qt = p.n_qtiles - 1 - blockIdx.z / p.max_splits;
+  const int kv_begin = split * p.split_len;
+  int q_start, q_len, L, q_raw;
+  seq_geometry_uniform(p, seq, q_start, q_len, L, &q_raw);
+  const int j0 = qt * p.qtile;
+  const int jn = (q_len - j0 < p.qtile) ? q_len - j0 : p.qtile;
+  const int kv_limit = L - q_len + j0 + jn;  // meaningful when jn > 0
+  const int nsplit = kv_limit > 0 ? (kv_limit + p.split_len - 1) / p.split_len : 0;
+  const bool note = kvh == 0 && split == 0 && p.row_nsplit;
+  const bool clip_owner = kvh == 0 && split == 0 && qt == p.n_qtiles - 1 && q_raw > q_len;
+  if (jn <= 0 || kv_begin >= kv_limit) {
+    if (jn > 0) {
+      if (note) note_rows(p, seq, qt, nsplit);
+      if (kv_limit <= 0 && split == 0) zero_tile(p, kvh, seq, qt);
+    }
+    if (clip_owner) clear_clipped_rows(p, q_start, q_len, q_raw, threadIdx.x, blockDim.x);
+    return;
+  }
+  if (note) note_rows(p, seq, qt, nsplit);
+  const int kv_end = kv_begin + p.split_len < kv_limit ? kv_begin + p.split_len : kv_limit;
+
+  const int tid = threadIdx.x % kThreads;
+  const int lane = tid & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads) : 0;
+  uint32_t* const bufs = lds + kg * 2 * kWideBuf;
+  const int h = lane >> 5;
+  const int col = lane & 31;
+  const int rows = jn * p.group;
+  float kscale = 1.0f, vscale = 1.0f;
+  if (FP8) {
+    kscale = p.k_scale ? *p.k_scale : 1.0f;
+    vscale = p.v_scale ? *p.v_scale : 1.0f;
+  }
+  const float sl2 = p.scale_log2 * kscale;
+
+  // ---- this lane's query column (a padding column repeats row 0 and is
+  // masked), its causal limit, and the wave's first and last limits
+  const int n = 32 * wv + col;
+  const int nn = n < rows ? n : 0;
+  const int jc = j0 + nn / p.group, hc = kvh * p.group + nn % p.group;
+  bf16x8_t qv[8];
+  {
+    const uint16_t* qp = p.q + static_cast<int64_t>(q_start + jc) * p.q_row_stride +
+                         static_cast<int64_t>(hc) * p.q_head_stride + 8 * h;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) qv[s] = *reinterpret_cast<const bf16x8_t*>(qp + 16 * s);
+  }
+  const int lim = n < rows ? L - q_len + jc : -1;
+  // keys below wave_full are visible to every row of the wave, keys at or
+  // past wave_end to none
+  const int first_row = 32 * wv < rows ? 32 * wv : rows - 1;
+  const int last_row = 32 * wv + 31 < rows ? 32 * wv + 31 : rows - 1;
+  const int wave_full = 32 * wv + 31 < rows ? L - q_len + j0 + first_row / p.group + 1 : 0;
+  const int wave_end = 32 * wv < rows ? L - q_len + j0 + last_row / p.group + 1 : 0;
+
+  // ---- loads: thread granule i is row (tid + i kThreads) / kRowGran of the
+  // tile; its 32-key half is the same for the whole wave.  The two halves
+  // have descriptors of their own (blocks hold a multiple of 32 tokens),
+  // which end at the last visible key.
+  const uint32_t tokb = static_cast<uint32_t>(p.tok_stride * kEsz);
+  constexpr int kStepRows = kThreads / kRowGran;         // rows between a thread's granules
+  uint32_t goff[kPer], kdst[kPer], vdst[kPer];
+  bool upper[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int gi = tid + i * kThreads;
+    const int row = gi / kRowGran, c = gi % kRowGran;
+    upper[i] = kStepRows <= 32 ? i * kStepRows >= 32 : __builtin_amdgcn_readfirstlane(row) >= 32;
+    goff[i] = static_cast<uint32_t>(row & 31) * tokb + c * 16;
+    kdst[i] = row * kWideKPitch + c * (FP8 ? 8 : 4);
+    vdst[i] = kWideKeys * kWideKPitch + row * kWideVPitch + c * (FP8 ? 8 : 4);
+  }
+  // lane i of lane_blk holds the id of the logical block i past the one that
+  // ld_blk counts from
+  const int first_blk = kv_begin / p.block_size;
+  int lane_blk = split_block_ids(p, seq, kv_begin);
+  int ld_key = kv_begin;                            // first key of the next half to load,
+  int ld_blk = 0;                                   // its block
+  int ld_tok = kv_begin - first_blk * p.block_size; // and its token there
+  auto advance_half = [&] {                         // blocks hold a multiple of 32 tokens
+    ld_key += 32;
+    ld_tok += 32;
+    if (ld_tok == p.block_size) {
+      ld_tok = 0;
+      ++ld_blk;
+    }
+  };
+  for (int i = 0; i < 2 * kg; ++i) advance_half();
+  // the next 32-key half: its descriptors, and whether its block is valid
+  auto next_half = [&](__amdgpu_buffer_rsrc_t& kr, __amdgpu_buffer_rsrc_t& vr) -> bool {
+    const bool live = ld_key < kv_end;
+    if (live && ld_blk >= kWave) {
+      ld_blk = 0;
+      lane_blk = split_block_ids(p, seq, ld_key);
+    }
+    const int raw = __builtin_amdgcn_readlane(lane_blk, ld_blk & (kWave - 1));
+    const bool valid = live && raw >= 0 && raw < p.num_blocks;
+    const int visible = kv_limit - ld_key < 32 ? kv_limit - ld_key : 32;
+    const int nrec = valid ? visible * static_cast<int>(tokb) : 0;
+    const int64_t tile = (static_cast<int64_t>(valid ? raw : 0) * p.blk_stride +
+                          static_cast<int64_t>(kvh) * p.head_stride +
+                          static_cast<int64_t>(valid ? ld_tok : 0) * p.tok_stride) * kEsz;
+    kr = make_rsrc(p.k_cache + tile, nrec);
+    vr = make_rsrc(p.v_cache + tile, nrec);
+    advance_half();
+    return valid;
+  };
+  struct Tile {
+    uint4 k[kPer], v[kPer];
+    int valid;                                      // bit 0, 1: the halves
+  };
+  auto load_tile = [&](Tile& t) {
+    __amdgpu_buffer_rsrc_t k0, v0, k1, v1;
+    const bool a = next_half(k0, v0);
+    const bool b = next_half(k1, v1);
+    t.valid = (a ? 1 : 0) | (b ? 2 : 0);
+#pragma unroll
+    for (int i = 0; i < 2 * (KG - 1); ++i) advance_half();   // the other group's tile
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      t.k[i] = __builtin_bit_cast(
+          uint4, __builtin_amdgcn_raw_buffer_load_b128(upper[i] ? k1 : k0, goff[i], 0, 0));
+      t.v[i] = __builtin_bit_cast(
+          uint4, __builtin_amdgcn_raw_buffer_load_b128(upper[i] ? v1 : v0, goff[i], 0, 0));
+    }
+  };
+  auto stage = [&](const Tile& t, int b) {
+    uint32_t* base = bufs + b * kWideBuf;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      if constexpr (FP8) {
+        *reinterpret_cast<bf16x8_t*>(base + kdst[i]) = fp8x8_to_bf16(make_uint2(t.k[i].x, t.k[i].y));
+        *reinterpret_cast<bf16x8_t*>(base + kdst[i] + 4) = fp8x8_to_bf16(make_uint2(t.k[i].z, t.k[i].w));
+        *reinterpret_cast<bf16x8_t*>(base + vdst[i]) = fp8x8_to_bf16(make_uint2(t.v[i].x, t.v[i].y));
+        *reinterpret_cast<bf16x8_t*>(base + vdst[i] + 4) = fp8x8_to_bf16(make_uint2(t.v[i].z, t.v[i].w));
+      } else {
+        *reinterpret_cast<uint4*>(base + kdst[i]) = t.k[i];
+        *reinterpret_cast<uint4*>(base + vdst[i]) = t.v[i];
+      }
+    }
+  };
+
+  float m_run = -INFINITY, l_run = 0.0f;
+  f32x16_t acc[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[dt][i] = 0.0f;
+
+  auto compute = [&](int kb, int valid, int b) {
+    if (kb >= wave_end || valid == 0) return;
+    const uint32_t* kst = bufs + b * kWideBuf;
+    const uint32_t* vst = kst + kWideKeys * kWideKPitch;
+    f32x16_t sacc[2];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sacc[kt][i] = 0.0f;
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        const bf16x8_t ko =
+            *reinterpret_cast<const bf16x8_t*>(kst + (32 * kt + col) * kWideKPitch + 8 * s + 4 * h);
+        sacc[kt] = mfma32(ko, qv[s], sacc[kt]);
+      }
+    if (kb + kWideKeys > wave_full || valid != 3) {
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int key = kb + 32 * kt + 8 * (i >> 2) + 4 * h + (i & 3);
+          if (key > lim || !((valid >> kt) & 1)) sacc[kt][i] = -INFINITY;
+        }
+    }
+    float cmax = sacc[0][0];
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) cmax = fmaxf(cmax, sacc[kt][i]);
+    cmax = max_xor32(cmax) * sl2;
+    const bool need = cmax > m_run + kRescaleSlack;
+    if (__any(need)) {
+      const float m_new = need ? cmax : m_run;
+      const float alpha = need ? exp2f_fast(m_run - m_new) : 1.0f;
+      l_run *= alpha;
+      m_run = m_new;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[dt][i] *= alpha;
+    }
+    const float msub = m_run == -INFINITY ? 0.0f : m_run;
+    bf16x8_t pb[4];
+    float psum[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      uint32_t w[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        f32x2_t pv;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          pv[e] = exp2f_fast(__builtin_fmaf(sacc[t >> 1][8 * (t & 1) + 2 * j + e], sl2, -msub));
+          psum[e] += pv[e];
+        }
+        w[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pv, bf16x2_t));
+      }
+      pb[t] = __builtin_bit_cast(bf16x8_t, make_uint4(w[0], w[1], w[2], w[3]));
+    }
+    l_run += psum[0] + psum[1];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) acc[dt] = mfma32(wide_v_operand(vst, lane, t, dt), pb[t], acc[dt]);
+
+  };
+
+  // step c computes tile c from buffer c & 1, stages tile c + 1 into the other
+  // buffer and loads tile c + 2; the barrier publishes the staged tile and
+  // frees the computed one
+  const int ntiles = (kv_end - kv_begin + KG * kWideKeys - 1) / (KG * kWideKeys);
+  Tile t;
+  load_tile(t);
+  stage(t, 0);
+  int valid = t.valid;
+  load_tile(t);
+  __syncthreads();
+  for (int c = 0; c < ntiles; ++c) {
+    compute(kv_begin + (c * KG + kg) * kWideKeys, valid, c & 1);
+    if (c + 1 < ntiles) {
+      stage(t, (c + 1) & 1);
+      valid = t.valid;
+      load_tile(t);
+    }
+    __syncthreads();
+  }
+
+  // ---- finish: elements 4 b + i of tile dt are d = 32 dt + 8 b + 4 h + i;
+  // exchanging between the lane halves gives each lane eight consecutive ones
+  if constexpr (KG > 1) {
+    // the other key group's waves park their states (every buffer is free
+    // behind the loop's last barrier) and this group's take them in
+    static_assert(KG == 2, "one merge");
+    float* park = reinterpret_cast<float*>(lds) + wv * kWave * 66;
+    if (kg == 1) {
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+          reinterpret_cast<f32x4_t*>(park)[(4 * dt + b) * kWave + lane] =
+              f32x4_t{acc[dt][4 * b], acc[dt][4 * b + 1], acc[dt][4 * b + 2], acc[dt][4 * b + 3]};
+      park[64 * kWave + lane] = m_run;
+      park[65 * kWave + lane] = l_run;
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float m1 = park[64 * kWave + lane], l1 = park[65 * kWave + lane];
+    const float M = fmaxf(m_run, m1);
+    const float f0 = m_run == -INFINITY ? 0.0f : exp2f_fast(m_run - M);
+    const float f1 = m1 == -INFINITY ? 0.0f : exp2f_fast(m1 - M);
+    m_run = M;
+    l_run = f0 * l_run + f1 * l1;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const f32x4_t o = reinterpret_cast<const f32x4_t*>(park)[(4 * dt + b) * kWave + lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[dt][4 * b + i] = f0 * acc[dt][4 * b + i] + f1 * o[i];
+      }
+  }
+  const float lsum = sum_xor32(l_run);
+  const float inv = lsum > 0.0f ? vscale / lsum : 0.0f;
+  if (n < rows) {
+    const int64_t tok = q_start + jc;
+    const int64_t slot = (tok * p.hq + hc) * p.max_splits + split;
+    if (nsplit == 1) {
+      uint16_t* op = p.out + tok * p.out_row_stride + static_cast<int64_t>(hc) * p.out_head_stride;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int b = 0; b < 4; b += 2) {
+          uint32_t w[2][2];
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+              w[e][k] = pack_bf16(acc[dt][4 * (b + e) + 2 * k] * inv, acc[dt][4 * (b + e) + 2 * k + 1] * inv);
+          const auto r0 = __builtin_amdgcn_permlane32_swap(w[0][0], w[1][0], false, false);
+          const auto r1 = __builtin_amdgcn_permlane32_swap(w[0][1], w[1][1], false, false);
+          const uint32_t a0 = r0[0], a1 = r1[0], b0 = r0[1], b1 = r1[1];
+          *reinterpret_cast<uint4*>(op + 32 * dt + 8 * (b + h)) = make_uint4(a0, a1, b0, b1);
+        }
+    } else {
+      float* wo = p.ws_o + slot * kD;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+          *reinterpret_cast<float4*>(wo + 32 * dt + 8 * b + 4 * h) =
+              make_float4(acc[dt][4 * b] * inv, acc[dt][4 * b + 1] * inv, acc[dt][4 * b + 2] * inv,
+                          acc[dt][4 * b + 3] * inv);
+      if (h == 0) p.ws_lse[slot] = lsum > 0.0f ? m_run + __log2f(lsum) : -INFINITY;
     }
   }
   if (clip_owner) clear_clipped_rows(p, q_start, q_len, q_raw, threadIdx.x, blockDim.x);
@@ -1265,12 +1631,11 @@ paged_attention_stream_kernel(AttnParams p) {
       const int c1 = (end < hi ? end : hi) - lo;
       int q_start, q_len, L;
       seq_geometry_uniform(p, s, q_start, q_len, L);
-      const int kv_limit = L;
       const int kv_begin = c0 * kChunk;
-      const int kv_end = c1 * kChunk < kv_limit ? c1 * kChunk : kv_limit;
+      const int kv_end = c1 * kChunk < L ? c1 * kChunk : L;
       const int split = r - lo / rc;
       const int nsplit = (hi - 1) / rc - lo / rc + 1;
-      attend_segment<NT, FP8, PIPE, 1>(p, vst, qst, kvh, s, 0, q_start, q_len, L, kv_begin, kv_end,
+      attend_segment<NT, FP8, PIPE, 1>(p, vst, qst, kvh, s, q_start, q_len, L, kv_begin, kv_end,
                                        split, nsplit, split_block_ids(p, s, kv_begin));
     }
   }
@@ -1355,7 +1720,7 @@ int32_t device_cus() {
 }
 
 // Split length of the fixed decomposition.  A segment is one (sequence, kv
-// head, query tile); `waves` waves share each split.
+// head); `waves` waves share each split.
 //   * Eight waves per split (bf16 tiles of up to 32 rows): 352 keys per
 //     wave, 2816 per split; when the batch has at least four segments per
 //     CU (several rounds of workgroups, which the dispatcher balances), one
@@ -1383,10 +1748,10 @@ int32_t device_cus() {
 // (the kernel holds one block id per lane); block_size 0 (unknown: the
 // workspace query) assumes the smallest block, kChunk tokens, which bounds
 // the split count from above.
-void choose_split(int32_t num_seqs, int32_t num_kv_heads, int32_t n_qtiles, int32_t max_k,
-                  int32_t waves, int32_t block_size, int32_t* split_len, int32_t* max_splits) {
+void choose_split(int32_t num_seqs, int32_t num_kv_heads, int32_t max_k, int32_t waves,
+                  int32_t block_size, int32_t* split_len, int32_t* max_splits) {
   const int64_t segs = static_cast<int64_t>(num_seqs > 0 ? num_seqs : 1) *
-                       (num_kv_heads > 0 ? num_kv_heads : 1) * (n_qtiles > 0 ? n_qtiles : 1);
+                       (num_kv_heads > 0 ? num_kv_heads : 1);
   const int64_t base = segs * (waves > 0 ? waves : 1);
   const int32_t mk = max_k > 1 ? max_k : 1;
   const int32_t cus = device_cus();
@@ -1495,9 +1860,9 @@ int tile_mfmas(int32_t tile_rows) { return tile_rows <= 16 ? 1 : tile_rows <= 32
 // Up to kPairedMaxKeys keys per sequence (the shapes measured);
 // NVA_ATTN_PAIRED=0/1 overrides the choice (tuning).
 constexpr int32_t kPairedMaxKeys = 3072;
-bool paired_mode(int32_t num_seqs, int32_t hkv, int32_t n_qtiles, int32_t max_k, int nt, bool fp8) {
+bool paired_mode(int32_t num_seqs, int32_t hkv, int32_t max_k, int nt, bool fp8) {
   static const int forced = env_choice("NVA_ATTN_PAIRED");
-  if (forced == 0 || fp8 || nt != 2 || n_qtiles != 1 || pipelined(nt, fp8)) return false;
+  if (forced == 0 || fp8 || nt != 2 || pipelined(nt, fp8)) return false;
   if (max_k > kPairedMaxKeys) return false;
   const int64_t segs = static_cast<int64_t>(num_seqs) * hkv;
   const int64_t cus = device_cus();
@@ -1522,6 +1887,58 @@ int32_t stream_ranges_per_head(int32_t hkv) {
   return (simds + h - 1) / h;
 }
 
+// The wide-tile kernel's launch for sequences of several 64-row query tiles.
+// `groups` bounds the workgroups of 128 rows (a sequence has at most one part
+// tile).  Measured on MI355X, one prompt of L tokens unless said otherwise, us:
+//   * two key groups (eight waves, one workgroup a CU) where four-wave
+//     workgroups would leave CUs empty or alone: a workgroup by itself takes
+//     ~1.5 us a 64-key step, two key groups share the steps.  Qwen3-0.6B
+//     L 1024 (128 groups) 31.4 -> 25.6, L 4096 (512) 119 -> 92; Qwen3-8B
+//     L 1024 (256) 32.3 -> 26.7, L 2048 (512) 63.7 -> 53.9.  Past one group a
+//     CU only for long key ranges: 3 x 300 tokens at Qwen3-32B (480) 18.0
+//     against 23.9; past two a CU it loses (1024 groups: 95 against 102).
+//   * eight waves sharing each K/V tile for long sequences, where the start-up
+//     of the wider workgroup is a small part: 16384 tokens as 8192-token
+//     prompts at Qwen3-8B 1129 -> 1091, 4096-token ones 606 -> 582,
+//     Qwen3-0.6B FP8 316 -> 300; short ones stay at four (256-2048 tokens,
+//     FP8 0.6B, 129 against 151).
+//   * key splits while there are fewer groups than CUs (a verify of more than
+//     64 rows over long contexts): 72 rows over 16000 keys 29 us split against
+//     ~240 whole (8 groups), 55 with the 64-row tiles.
+struct WidePlan {
+  int32_t waves, key_groups, qtile, n_qtiles, split_len, max_splits;
+};
+WidePlan wide_plan(int32_t num_seqs, int32_t num_tokens, int32_t hkv, int32_t group, int32_t max_q,
+                   int32_t max_k) {
+  WidePlan w;
+  const int64_t cus = device_cus();
+  const int32_t mk = max_k > 1 ? max_k : 1;
+  const int64_t rows = static_cast<int64_t>(num_tokens) * group;
+  const int64_t per_seq = (static_cast<int64_t>(max_q) * group + 127) / 128;
+  int64_t tiles = rows / 128 + num_seqs;
+  if (num_seqs * per_seq < tiles) tiles = num_seqs * per_seq;
+  const int64_t groups = tiles * hkv;
+  w.waves = 4;
+  w.key_groups = 1;
+  if (groups <= cus || (groups <= 2 * cus && mk >= 1024))
+    w.key_groups = 2;
+  else if (rows >= 8192 * static_cast<int64_t>(num_seqs))
+    w.waves = 8;
+  w.qtile = 32 * w.waves / group;
+  w.n_qtiles = (max_q + w.qtile - 1) / w.qtile;
+  const int64_t parts = groups < cus ? cus / groups : 1;
+  const int64_t len = (mk + parts - 1) / parts;
+  w.split_len = static_cast<int32_t>((len + kMinSplit - 1) / kMinSplit * kMinSplit);
+  w.max_splits = (mk + w.split_len - 1) / w.split_len;
+  return w;
+}
+
+size_t partials_bytes(int32_t num_tokens, int32_t hq, int32_t max_splits) {
+  const size_t slots = static_cast<size_t>(num_tokens) * hq * max_splits;
+  return slots * kD * sizeof(float) + slots * sizeof(float) +
+         static_cast<size_t>(num_tokens) * sizeof(int32_t) + 256;
+}
+
 // Workspace for either KV dtype (the size query does not name one): the
 // larger of the stream and fixed layouts that could apply to either.
 size_t workspace_bytes(int32_t num_seqs, int32_t num_tokens, int32_t hq, int32_t hkv, int32_t max_q,
@@ -1531,21 +1948,22 @@ size_t workspace_bytes(int32_t num_seqs, int32_t num_tokens, int32_t hq, int32_t
   size_t bytes = 0;
   if (stream_mode(num_seqs, max_q, qtile, group, false) ||
       stream_mode(num_seqs, max_q, qtile, group, true)) {
-    const size_t slots = static_cast<size_t>(num_tokens) * hq * stream_max_splits(max_k);
-    bytes = slots * kD * sizeof(float) + slots * sizeof(float) +
-            static_cast<size_t>(num_tokens) * sizeof(int32_t) + 512;
+    bytes = partials_bytes(num_tokens, hq, stream_max_splits(max_k));
   }
   const int32_t n_qtiles = (max_q + qtile - 1) / qtile;
+  if (n_qtiles > 1) {
+    if (group < 1 || group > 64) return 0;   // refused at the launch
+    const WidePlan w = wide_plan(num_seqs, num_tokens, hkv, group, max_q, max_k);
+    return w.max_splits > 1 ? partials_bytes(num_tokens, hq, w.max_splits) : 0;
+  }
   const int nt = tile_mfmas(qtile * (hkv > 0 ? hq / hkv : 1));
   // either KV dtype: the larger split count of the two wave choices
   int32_t len, ms, ms_fp8;
-  choose_split(num_seqs, hkv, n_qtiles, max_k, segment_waves(nt, false), 0, &len, &ms);
-  choose_split(num_seqs, hkv, n_qtiles, max_k, segment_waves(nt, true), 0, &len, &ms_fp8);
+  choose_split(num_seqs, hkv, max_k, segment_waves(nt, false), 0, &len, &ms);
+  choose_split(num_seqs, hkv, max_k, segment_waves(nt, true), 0, &len, &ms_fp8);
   ms = ms_fp8 > ms ? ms_fp8 : ms;
   if (ms > 1) {
-    const size_t slots = static_cast<size_t>(num_tokens) * hq * ms;
-    const size_t fixed = slots * kD * sizeof(float) + slots * sizeof(float) +
-                         static_cast<size_t>(num_tokens) * sizeof(int32_t) + 256;
+    const size_t fixed = partials_bytes(num_tokens, hq, ms);
     bytes = fixed > bytes ? fixed : bytes;
   }
   return bytes;
@@ -1651,6 +2069,14 @@ void launch_nt(const AttnParams& p, bool fp8, bool stream, int wps, dim3 grid, h
     paged_attention_kernel<NT, false, false, 1><<<grid, kWave, 0, s>>>(p);
 }
 
+template <int NW, int KG>
+void launch_wide(const AttnParams& p, bool fp8, dim3 grid, hipStream_t s) {
+  if (fp8)
+    paged_attention_wide_kernel<NW, KG, true><<<grid, NW * KG * kWave, 0, s>>>(p);
+  else
+    paged_attention_wide_kernel<NW, KG, false><<<grid, NW * KG * kWave, 0, s>>>(p);
+}
+
 int run_attention(AttnParams& p, int kv_dtype, void* workspace, size_t workspace_bytes_, hipStream_t s) {
   if (p.hq <= 0 || p.hkv <= 0 || p.hq % p.hkv != 0) return NVA_ERR_ARG;
   if (kv_dtype != NVA_KV_BF16 && kv_dtype != NVA_KV_FP8_E4M3) return NVA_ERR_ARG;
@@ -1671,18 +2097,28 @@ int run_attention(AttnParams& p, int kv_dtype, void* workspace, size_t workspace
       p.blk_stride % vec_elems || p.tok_stride % vec_elems || p.head_stride % vec_elems)
     return NVA_ERR_UNSUPPORTED;
   const bool fp8 = kv_dtype == NVA_KV_FP8_E4M3;
+  const bool wide = p.n_qtiles > 1;
   const bool stream = stream_mode(p.num_seqs, p.max_q, p.qtile, p.group, fp8);
   const int nt = tile_mfmas(tile_rows);
   // paired mode's whole-sequence split must fit the kernel's block ids
   const int32_t mk = p.max_k > 1 ? p.max_k : 1;
   const int32_t whole = (mk + kMinSplit - 1) / kMinSplit * kMinSplit;
-  const bool paired = !stream && paired_mode(p.num_seqs, p.hkv, p.n_qtiles, p.max_k, nt, fp8) &&
+  const bool paired = !wide && !stream && paired_mode(p.num_seqs, p.hkv, p.max_k, nt, fp8) &&
                       whole / p.block_size + 2 <= kWave;
-  int wps = segment_waves(nt, fp8);
+  int wps = segment_waves(nt, fp8), key_groups = 1;
   dim3 grid;
   p.row_nsplit = nullptr;
   p.pair_rows = 0;
-  if (stream) {
+  if (wide) {
+    const WidePlan w = wide_plan(p.num_seqs, p.num_tokens, p.hkv, p.group, p.max_q, p.max_k);
+    wps = w.waves;
+    key_groups = w.key_groups;
+    p.qtile = w.qtile;
+    p.n_qtiles = w.n_qtiles;
+    p.split_len = w.split_len;
+    p.max_splits = w.max_splits;
+    grid = dim3(p.hkv, p.num_seqs, p.max_splits * p.n_qtiles);
+  } else if (stream) {
     // a range may span at most kWave - 2 whole blocks (one block id per lane)
     p.min_range_chunks = kMinRangeChunks;
     p.max_range_chunks = (kWave - 2) * p.block_size / kChunk;
@@ -1695,13 +2131,13 @@ int run_attention(AttnParams& p, int kv_dtype, void* workspace, size_t workspace
     p.split_len = whole;
     p.max_splits = 1;
     p.pair_rows = device_cus() / p.hkv;
-    grid = dim3(p.hkv, p.num_seqs, p.n_qtiles);
+    grid = dim3(p.hkv, p.num_seqs, 1);
   } else {
-    choose_split(p.num_seqs, p.hkv, p.n_qtiles, p.max_k, wps, p.block_size, &p.split_len,
+    choose_split(p.num_seqs, p.hkv, p.max_k, wps, p.block_size, &p.split_len,
                  &p.max_splits);
     // the kernel keeps one block id per lane: a split may touch at most kWave blocks
     if (p.split_len / p.block_size + 2 > kWave) return NVA_ERR_UNSUPPORTED;
-    grid = dim3(p.hkv, p.num_seqs, p.max_splits * p.n_qtiles);
+    grid = dim3(p.hkv, p.num_seqs, p.max_splits);
   }
   if (stream || p.max_splits > 1) {
     const size_t need = workspace_bytes(p.num_seqs, p.num_tokens, p.hq, p.hkv, p.max_q, p.max_k);
@@ -1718,7 +2154,13 @@ int run_attention(AttnParams& p, int kv_dtype, void* workspace, size_t workspace
     p.ws_o = nullptr;
     p.ws_lse = nullptr;
   }
-  if (nt <= 1)
+  if (wide && key_groups == 2)
+    launch_wide<4, 2>(p, fp8, grid, s);
+  else if (wide && wps == 8)
+    launch_wide<8, 1>(p, fp8, grid, s);
+  else if (wide)
+    launch_wide<4, 1>(p, fp8, grid, s);
+  else if (nt <= 1)
     launch_nt<1>(p, fp8, stream, wps, grid, s);
   else if (nt == 2)
     launch_nt<2>(p, fp8, stream, wps, grid, s);

@@ -1147,3 +1147,64 @@ def test_draft_metadata_after_verify(K, cuda):
         np.testing.assert_array_equal(pos.cpu().numpy(), opos)
         np.testing.assert_array_equal(slots.cpu().numpy(), oslots)
         np.testing.assert_array_equal(ctx.cpu().numpy(), octx)
+
+
+WIDE_CASES = [
+    # every tile edge of the wide-tile kernel: query rows around 128 and 256
+    # (positions times group), keys around its 64-key step, rows equal to keys
+    # (a prompt) and fewer (cached prefix), a sequence without rows
+    ("tile_edges", dict(q_len=[65, 33, 64, 63, 0, 1, 17, 128, 129], ctx_lo=1, ctx_hi=300, hq=16, hkv=4,
+                        block_size=32)),
+    ("one_prompt", dict(q_len=[700], ctx_lo=700, ctx_hi=700, hq=16, hkv=8)),
+    ("cached_prefix", dict(q_len=[70, 41], ctx_lo=900, ctx_hi=1100, hq=32, hkv=8, block_size=32)),
+    # few workgroups over many keys: key splits, then the combine
+    ("split_keys", dict(q_len=[9, 9], ctx_lo=3900, ctx_hi=4200, hq=64, hkv=8)),
+    # as many query rows as pick the 256-row workgroups
+    ("eight_waves", dict(q_len=[257], ctx_lo=290, ctx_hi=290, hq=128, hkv=4)),
+    # groups that do not divide a tile
+    ("group3", dict(q_len=[150, 22, 90], ctx_lo=100, ctx_hi=260, hq=12, hkv=4, block_size=32)),
+    ("group40", dict(q_len=[30, 7], ctx_lo=64, ctx_hi=193, hq=40, hkv=1)),
+    ("group1", dict(q_len=[300, 66], ctx_lo=66, ctx_hi=330, hq=8, hkv=8, block_size=32)),
+]
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("name,kw", WIDE_CASES, ids=[c[0] for c in WIDE_CASES])
+def test_several_query_tiles(K, cuda, name, kw, fp8):
+    """Sequences of several 64-row query tiles against the oracle.  The bound
+    is the verify tests': probabilities and outputs rounded to bf16."""
+    case = paged_case(seed=21, batch=len(kw["q_len"]), **kw)
+    got, ref = _run_verify(K, cuda, case, fp8=fp8, head_major="kv_adjacent")
+    err = np.abs(got - ref).max()
+    assert err <= ATTN_TOL, (name, err)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_several_query_tiles_skip_invalid_blocks_and_scale(K, cuda, fp8):
+    """Keys of a block id outside the cache are not seen by any query tile
+    (2500 keys in 32-token pages: more than the 64 block ids a wave holds at
+    once), and FP8 scales apply: equal to the oracle on the pages that are
+    left, whose tables hold only the valid blocks' keys."""
+    case = paged_case(seed=5, batch=1, q_len=[40], ctx_lo=2500, ctx_hi=2500, hq=16, hkv=4,
+                      block_size=32)
+    kc, vc = case["k_cache"], case["v_cache"]
+    if fp8:
+        kc, vc = kc.float().to(torch.float8_e4m3fn), vc.float().to(torch.float8_e4m3fn)
+    ks, vs = (0.5, 1.5) if fp8 else (1.0, 1.0)
+    scales = [torch.full((1,), x, device=cuda) for x in (ks, vs)] if fp8 else [None, None]
+    bt = case["block_tables"].clone()
+    bad = [3, 40, 64, 66]
+    for i, b in enumerate(bad):
+        bt[0, b] = -1 if i % 2 else kc.shape[0] + 7
+    out = K.paged_attention_varlen(case["q"].to(cuda), kc.to(cuda), vc.to(cuda),
+                                   case["cu_q"].to(cuda), case["cu_k"].to(cuda), 40, 2500,
+                                   128 ** -0.5, bt.to(cuda), k_scale=scales[0], v_scale=scales[1])
+    torch.cuda.synchronize()
+    nblk = -(-2500 // 32)
+    keep = [b for b in range(nblk) if b not in bad]
+    sub = case["block_tables"][:, keep].contiguous()
+    n = 2500 - 32 * len(bad)
+    ref = oracle.paged_attention(bits(case["q"]), bits(kc), bits(vc), case["cu_q"].numpy(),
+                                 np.array([n], np.int32), sub.numpy(), 128 ** -0.5, ks, vs)
+    err = np.abs(out.float().cpu().numpy() - ref).max()
+    assert err <= ATTN_TOL, err
