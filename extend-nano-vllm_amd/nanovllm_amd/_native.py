@@ -1,4 +1,5 @@
-"""ctypes binding of libnanovllm_amd.so (the C ABI in include/nanovllm_amd.h).
+"""ctypes binding of libnanovllm_amd.so (the C ABI in include/nanovllm_amd.h),
+and the loader of the native front end (lib/_front_end.so) over the same library.
 
 The library is built in-tree by extend-nano-vllm_amd/csrc/Makefile into
 nanovllm_amd/lib/.  There is no fallback: if the library is missing every
@@ -7,11 +8,14 @@ kernel call raises ``NativeLibraryError``.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import subprocess
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG, "lib", "libnanovllm_amd.so")
+FRONT_PATH = os.path.join(_PKG, "lib", "_front_end.so")
 CSRC_DIR = os.path.join(os.path.dirname(_PKG), "csrc")
 
 NVA_OK = 0
@@ -110,6 +114,28 @@ def load() -> ctypes.CDLL:
         fn.argtypes = argtypes
     _lib = lib
     return lib
+
+
+_front = None
+
+
+def load_front_end():
+    """The CPython module in front of the library (csrc/front_end.cpp)."""
+    global _front
+    if _front is None:
+        load()
+        if not os.path.exists(FRONT_PATH):
+            raise NativeLibraryError(f"{FRONT_PATH} is missing: build it with `make -C {CSRC_DIR}` "
+                                     "(or __graft_entry__.build())")
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("_front_end", FRONT_PATH)
+            spec = importlib.util.spec_from_loader("_front_end", loader)
+            module = importlib.util.module_from_spec(spec)
+            loader.exec_module(module)
+        except ImportError as exc:
+            raise NativeLibraryError(f"cannot load {FRONT_PATH}: {exc}") from exc
+        _front = module
+    return _front
 
 
 def check(status: int, what: str) -> None:

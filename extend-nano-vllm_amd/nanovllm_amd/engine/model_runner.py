@@ -63,7 +63,7 @@ class ModelRunner:
     def __init__(self, config, rank: int = 0, event=None):
         if rank != 0:
             raise ValueError("this build runs one process per GPU (rank 0 only)")
-        _native.load()   # fail loudly without the HIP library
+        _native.load_front_end()   # fail loudly without the HIP library
         self.config = config
         hf = config.hf_config
         self.block_size = config.kvcache_block_size
@@ -129,7 +129,9 @@ class ModelRunner:
                 self._state_slot: dict[int, int] = {}
                 self._free_state = list(range(rows - 1, -1, -1))
         finally:
-            torch.set_default_device("cpu")
+            # not "cpu": a default device that is set, whichever, sends every
+            # later torch call through a Python mode
+            torch.set_default_device(None)
             torch.set_default_dtype(default_dtype)
         # benchmarks may ask to keep the last verify's logits and inputs, or to
         # run the verify forward eagerly (kernel-level timing)

@@ -9,6 +9,12 @@ reserved before capture, see ``reserve_workspace``).
 
 There is no CPU or PyTorch fallback: without the HIP library (or without a
 GPU) these functions raise.
+
+The functions a layer calls go through the native front end first
+(``_native.load_front_end``): it makes the same checks and the same call in
+~2-4 us, and answers None, having done nothing, for arguments that are not of
+the ordinary form; the code below then takes the call or raises.  Host time of
+one Qwen3-8B layer's nine calls: ~300 us without it.
 """
 from __future__ import annotations
 
@@ -21,6 +27,15 @@ from ._native import check
 
 BF16 = torch.bfloat16
 FP8 = torch.float8_e4m3fn
+
+
+_front = None
+
+
+def _front_end():
+    global _front
+    _front = _native.load_front_end()
+    return _front
 
 
 def _stream() -> int:
@@ -74,12 +89,13 @@ class _Workspaces:
     at them."""
 
     def __init__(self) -> None:
-        self._bufs: dict[tuple[int, str], torch.Tensor] = {}
+        self._bufs: dict[str, dict[int, torch.Tensor]] = {"argmax": {}, "attention": {}}
         self._retired: list[torch.Tensor] = []
 
     def get(self, device: torch.device, kind: str, nbytes: int) -> torch.Tensor:
-        key = (device.index if device.index is not None else torch.cuda.current_device(), kind)
-        buf = self._bufs.get(key)
+        key = device.index if device.index is not None else torch.cuda.current_device()
+        bufs = self.of(kind)
+        buf = bufs.get(key)
         if buf is None or buf.numel() < nbytes:
             if torch.cuda.is_current_stream_capturing():
                 raise RuntimeError(
@@ -89,11 +105,17 @@ class _Workspaces:
                 self._retired.append(buf)
                 size = max(size, 2 * buf.numel())
             buf = torch.zeros(size, dtype=torch.uint8, device=device)
-            self._bufs[key] = buf
+            bufs[key] = buf
         return buf
+
+    def of(self, kind: str) -> dict[int, torch.Tensor]:
+        """The buffers of one kind by device index."""
+        return self._bufs.setdefault(kind, {})
 
 
 _WS = _Workspaces()
+_ARGMAX_WS = _WS.of("argmax")
+_ATTENTION_WS = _WS.of("attention")
 
 
 def reserve_workspace(device: torch.device, kind: str, nbytes: int) -> None:
@@ -313,6 +335,9 @@ def argmax_rows(logits: torch.Tensor, index_map: torch.Tensor | None = None,
 
     Replaces Eagle3ForCausalLM.sample_greedy (eagle3.py:294-296, index_map =
     d2t) and Sampler's temperature-0 branch (sampler.py:10-19)."""
+    got = (_front or _front_end()).argmax_rows(logits, index_map, out, _ARGMAX_WS)
+    if got is not None:
+        return got
     lib = _native.load()
     _require_cuda(logits, index_map, out)
     if logits.dtype != BF16 or logits.dim() != 2 or logits.stride(1) != 1:
@@ -403,6 +428,11 @@ def paged_attention_varlen(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     a bound below them raises ValueError; device tensors are not read."""
     if not causal:
         raise ValueError("only causal paged attention is supported")
+    got = (_front or _front_end()).paged_attention_varlen(
+        q, k_cache, v_cache, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale,
+        block_table, k_scale, v_scale, out, _ATTENTION_WS)
+    if got is not None:
+        return got
     lib = _native.load()
     _require_cuda(q, k_cache, v_cache, block_table, out)
     cu_seqlens_q, host_q = _device_lengths(cu_seqlens_q, q.device, "cu_seqlens_q")
@@ -454,6 +484,11 @@ def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     lengths (default: every cache slot of one table row); the kernel clips a
     longer length to it.  When ``cache_seqlens`` is given on the host (a CPU
     tensor or a list) a bound below its largest value raises ValueError."""
+    got = (_front or _front_end()).paged_attention_decode(
+        q, k_cache, v_cache, cache_seqlens, block_table, softmax_scale, max_seqlen_k, k_scale,
+        v_scale, out, _ATTENTION_WS)
+    if got is not None:
+        return got
     lib = _native.load()
     _require_cuda(q, k_cache, v_cache, block_table, out)
     cache_seqlens, host_lens = _device_lengths(cache_seqlens, q.device, "cache_seqlens")
@@ -510,6 +545,9 @@ def _rows2d(x: torch.Tensor, name: str) -> None:
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float,
              out: torch.Tensor | None = None) -> torch.Tensor:
     """RMSNorm without residual (layers/layernorm.py:70-89)."""
+    got = (_front or _front_end()).rms_norm(x, weight, eps, out)
+    if got is not None:
+        return got
     lib = _native.load()
     _require_cuda(x, weight, out)
     _rows2d(x, "x")
@@ -529,6 +567,9 @@ def add_rms_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, 
     """RMSNorm with residual add (layers/layernorm.py:91-107).
 
     Returns (normed, new_residual); both are new tensors."""
+    got = (_front or _front_end()).add_rms_norm(x, residual, weight, eps)
+    if got is not None:
+        return got
     lib = _native.load()
     _require_cuda(x, residual, weight)
     _rows2d(x, "x")
@@ -544,6 +585,18 @@ def add_rms_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, 
     return out, res_out
 
 
+def merge_heads(x: torch.Tensor) -> torch.Tensor:
+    """[T, H, D] as [T, H * D]."""
+    got = (_front or _front_end()).merge_heads(x)
+    return x.reshape(x.shape[0], -1) if got is None else got
+
+
+def place(x: torch.Tensor) -> tuple:
+    """(device index, number of elements) of a tensor."""
+    got = (_front or _front_end()).place(x)
+    return (x.device.index, x.numel()) if got is None else got
+
+
 def _qkv_rows(qkv: torch.Tensor, positions: torch.Tensor, hq: int, hkv: int, d: int) -> None:
     if positions.numel() != qkv.shape[0]:
         raise ValueError("positions must have one entry per qkv row")
@@ -555,6 +608,9 @@ def add_then_rms_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Ten
     """``h = x + residual`` in bf16, then RMSNorm(h) without residual, as the
     EAGLE3 draft layer composes them (eagle3.py:141-146).  Returns
     (normed, h); both are new tensors."""
+    got = (_front or _front_end()).add_then_rms_norm(x, residual, weight, eps)
+    if got is not None:
+        return got
     lib = _native.load()
     _require_cuda(x, residual, weight)
     _rows2d(x, "x")
@@ -604,6 +660,11 @@ def qk_norm_rope_store(qkv: torch.Tensor, positions: torch.Tensor,
     heads of ``qkv`` (models/qwen3.py:77-98; attention.py:189-217), in one
     launch.  Returns q [T, Hq, D]; the cache contents are exactly those the
     two separate calls leave."""
+    got = (_front or _front_end()).qk_norm_rope_store(
+        qkv, positions, q_norm_weight, k_norm_weight, cos_sin, num_q_heads, num_kv_heads, head_dim,
+        eps, k_cache, v_cache, slot_mapping, k_scale, v_scale)
+    if got is not None:
+        return got
     lib = _native.load()
     _require_cuda(qkv, positions, q_norm_weight, k_norm_weight, cos_sin, k_cache, v_cache,
                   slot_mapping)
@@ -632,6 +693,9 @@ def qk_norm_rope_store(qkv: torch.Tensor, positions: torch.Tensor,
 
 def silu_mul(x: torch.Tensor) -> torch.Tensor:
     """SiluAndMul (layers/activation.py:11-14) on rows [a | b]."""
+    got = (_front or _front_end()).silu_mul(x)
+    if got is not None:
+        return got
     lib = _native.load()
     _require_cuda(x)
     _rows2d(x, "x")

@@ -116,7 +116,7 @@ class Attention(nn.Module):
         return self.attend(q)
 
     def _check_bound(self, ctx) -> None:
-        if not self.k_cache.numel():
+        if not K.place(self.k_cache)[1]:
             raise RuntimeError("attention needs a bound paged KV cache")
         if ctx.slot_mapping is None or ctx.block_tables is None:
             raise RuntimeError("paged KV attention requires slot mapping and block tables")
@@ -168,7 +168,7 @@ class SelfAttention(nn.Module):
     def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor) -> torch.Tensor:
         qkv = self.qkv_proj(hidden_states)
         cos_sin = rope_cos_sin(self.head_dim, self.max_position, float(self.rope_theta),
-                               qkv.device.index)
+                               K.place(qkv)[0])
         ctx = get_context()
         attn = self.attn
         if not ctx.is_dummy:
@@ -180,7 +180,7 @@ class SelfAttention(nn.Module):
                                      cos_sin, self.num_heads, self.num_kv_heads, self.head_dim,
                                      self.eps, attn.k_cache, attn.v_cache, ctx.slot_mapping,
                                      attn.k_scale, attn.v_scale)
-            return self.o_proj(attn.attend(q).view(-1, self.q_size))
+            return self.o_proj(K.merge_heads(attn.attend(q)))
         q, k = K.qk_norm_rope(qkv, positions,
                               self.q_norm.weight if self.use_qk_norm else None,
                               self.k_norm.weight if self.use_qk_norm else None,

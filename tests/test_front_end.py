@@ -1,0 +1,164 @@
+"""The native front end against the Python path behind it: bit-equal results
+for every form both take, and hands off (None) everything else."""
+import pytest
+import torch
+
+from nanovllm_amd import _native
+from nanovllm_amd import kernels as K
+
+BF16 = torch.bfloat16
+
+
+class _Absent:
+    """A front end that takes no call: the Python path alone."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+def test_hands_off_what_is_not_an_ordinary_gpu_call():
+    f = _native.load_front_end()
+    x, w = torch.zeros(2, 8, dtype=BF16), torch.ones(8, dtype=BF16)
+    assert f.rms_norm(x, w, 1e-6, None) is None                 # on the CPU
+    assert f.rms_norm(x.as_subclass(_Sub), w, 1e-6, None) is None
+    assert f.rms_norm(x.to("meta"), w.to("meta"), 1e-6, None) is None
+    assert f.rms_norm(None, w, 1e-6, None) is None
+    assert f.rms_norm(x, w, "eps", None) is None
+    assert f.add_rms_norm(x, x, w, 1) is None
+    assert f.silu_mul([1.0]) is None
+    assert f.place(x) is None and f.merge_heads(x) is None
+    with pytest.raises(TypeError):
+        f.rms_norm(x)
+
+
+def test_refusals_are_the_python_paths():
+    x = torch.zeros(2, 8, dtype=BF16)
+    with pytest.raises(ValueError, match="cuda"):
+        K.rms_norm(x, torch.ones(8), 1e-6)
+    with pytest.raises(ValueError, match="cuda"):
+        K.silu_mul(x)
+    with pytest.raises(ValueError, match="causal"):
+        K.paged_attention_varlen(x, x, x, x, x, 1, 1, 1.0, x, causal=False)
+    assert K.place(x) == (None, 16)
+    assert K.merge_heads(torch.zeros(2, 3, 4)).shape == (2, 12)
+
+
+def _both(monkeypatch, call):
+    """(through the front end, through the Python path); the front end must
+    have taken the call itself."""
+    front = _native.load_front_end()
+    taken = []
+
+    class Watch:
+        def __getattr__(self, name):
+            def fn(*args):
+                got = getattr(front, name)(*args)
+                taken.append(got is not None)
+                return got
+            return fn
+
+    monkeypatch.setattr(K, "_front", _Absent())
+    want = call()
+    monkeypatch.setattr(K, "_front", Watch())
+    got = call()
+    assert taken and all(taken)
+    return got, want
+
+
+def _same(got, want):
+    if isinstance(want, tuple):
+        assert len(got) == len(want)
+        for g, w in zip(got, want):
+            _same(g, w)
+        return
+    assert got.shape == want.shape and got.stride() == want.stride() and got.dtype == want.dtype
+    assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+def test_rows_equal_the_python_path(cuda, monkeypatch):
+    g = torch.Generator(device=cuda).manual_seed(3)
+    r = lambda *s: torch.randn(*s, generator=g, device=cuda).to(BF16)
+    w = r(200)
+    for x in (r(7, 200), r(7, 480)[:, 8:208], r(1, 200), r(9, 203)[:, 1:201], r(0, 200)):
+        y = r(*x.shape)
+        _same(*_both(monkeypatch, lambda: K.rms_norm(x, w, 1e-6)))
+        out = torch.empty(x.shape[0], 400, dtype=BF16, device=cuda)[:, 200:]
+        _same(*_both(monkeypatch, lambda: K.rms_norm(x, w, 1e-6, out=out).clone()))
+        _same(*_both(monkeypatch, lambda: K.add_rms_norm(x, y, w, 1e-6)))
+        _same(*_both(monkeypatch, lambda: K.add_then_rms_norm(x, y, w, 1e-6)))
+        _same(*_both(monkeypatch, lambda: K.silu_mul(x)))
+    table = torch.arange(1003, device=cuda) * 3
+    logits = r(6, 1003)
+    K.argmax_rows(logits)
+    for x, m in ((logits, None), (logits, table), (r(6, 1010)[:, :1003], table)):
+        _same(*_both(monkeypatch, lambda: K.argmax_rows(x, m)))
+        out = torch.zeros(9, dtype=torch.int64, device=cuda)
+        _same(*_both(monkeypatch, lambda: K.argmax_rows(x, m, out=out).clone()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("head_major", [False, True])
+def test_attention_equals_the_python_path(cuda, monkeypatch, fp8, head_major):
+    g = torch.Generator(device=cuda).manual_seed(4)
+    r = lambda *s: torch.randn(*s, generator=g, device=cuda).to(BF16)
+    hq, hkv, nb, bs = 8, 2, 11, 64
+    kv = r(nb, hkv, 2, bs, 128).permute(2, 0, 3, 1, 4) if head_major else r(2, nb, bs, hkv, 128)
+    kv = kv.to(torch.float8_e4m3fn) if fp8 else kv
+    one = torch.ones(1, device=cuda)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=cuda)
+    table = i32([[4, 9, 0, 2, 1], [7, 3, -1, -1, -1], [5, 6, 8, -1, -1]])
+    qkv = r(9, (hq + 2 * hkv) * 128 + 16)
+    qkv = qkv[:, : (hq + 2 * hkv) * 128]
+    pos = torch.tensor([5, 6, 7, 0, 3, 9, 10, 11, 12], device=cuda)
+    cos = torch.randn(64, 128, generator=g, device=cuda)
+    slots = i32([300, 301, 302, -1, 40, 500, 501, 502, nb * bs + 3])
+    k, v = kv[0].clone(), kv[1].clone()
+    norms = (r(128), r(128))
+    for qn, kn in (norms, (None, None)):
+        for ks, vs in ((None, None), (one * 0.5, one * 2)):
+            def store():
+                k.copy_(kv[0])
+                v.copy_(kv[1])
+                q = K.qk_norm_rope_store(qkv, pos, qn, kn, cos, hq, hkv, 128, 1e-6, k, v, slots, ks, vs)
+                return q, k.float(), v.float()
+            _same(*_both(monkeypatch, store))
+    k, v = kv[0], kv[1]                   # the layout's own strides
+    q = r(9, hq, 128)
+    for args in ((i32([0, 3, 4, 9]), i32([0, 300, 410, 600]), 5, 320),
+                 (i32([0, 1, 1, 9]), i32([0, 260, 270, 460]), 8, 300)):
+        for scales in ({}, dict(k_scale=one * 0.5, v_scale=one)):
+            varlen = lambda out=None: K.paged_attention_varlen(q, k, v, *args, 128 ** -0.5, table,
+                                                               out=out, **scales)
+            varlen()                      # the workspace is the Python path's to grow
+            _same(*_both(monkeypatch, varlen))
+            out = torch.zeros(9, hq, 256, dtype=BF16, device=cuda)[:, :, :128]
+            _same(*_both(monkeypatch, lambda: varlen(out).clone()))
+    lens = i32([310, 0, 190])
+    for bound in (None, 320):
+        decode = lambda: K.paged_attention_decode(q[:3], k, v, lens, table, 128 ** -0.5, bound,
+                                                  k_scale=one, v_scale=one)
+        decode()
+        _same(*_both(monkeypatch, decode))
+
+
+@pytest.mark.gpu
+def test_other_forms_still_run(cuda):
+    """Host lengths, a scale or bound of another number type: the Python path
+    takes them behind the front end."""
+    q = torch.randn(2, 4, 128, device=cuda).to(BF16)
+    kv = torch.randn(2, 2, 32, 2, 128, device=cuda).to(BF16)
+    table = torch.tensor([[0], [1]], dtype=torch.int32, device=cuda)
+    lens = torch.tensor([20, 31], dtype=torch.int32)
+    want = K.paged_attention_decode(q, kv[0], kv[1], lens.to(cuda), table, 0.5, 32)
+    import numpy as np
+    for n, s, b in ((lens, 0.5, 32), (lens.tolist(), 0.5, 32), (lens.to(cuda), np.float64(0.5), 32),
+                    (lens.to(cuda), 0.5, np.int64(32))):
+        assert torch.equal(K.paged_attention_decode(q, kv[0], kv[1], n, table, s, b), want)
+    with pytest.raises(ValueError):
+        K.paged_attention_decode(q, kv[0], kv[1], lens.tolist(), table, 0.5, 16)
