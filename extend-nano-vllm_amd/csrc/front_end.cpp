@@ -18,6 +18,11 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/PyInterpreter.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <limits>
 
@@ -414,6 +419,58 @@ PyObject* argmax_rows(PyObject*, PyObject* const* v, Py_ssize_t n) {
   });
 }
 
+// Whether something watches or rewrites torch calls (a function mode other than
+// the default device's, a dispatch mode, a tracer, autocast): those see the
+// Python path's calls.
+PyTypeObject* g_device_context = nullptr;   // torch.utils._device.DeviceContext
+bool watched() {
+  const int64_t modes = at::impl::PythonTorchFunctionTLS::stack_len();
+  for (int64_t i = 0; i < modes; ++i)
+    if (Py_TYPE(at::impl::PythonTorchFunctionTLS::get_stack_at(i)->ptr(getPyInterpreter())) !=
+        g_device_context)
+      return true;
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() || torch::jit::tracer::isTracing() ||
+         at::autocast::is_autocast_enabled(at::kCUDA);
+}
+
+struct WithoutGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
+// (x, weight, bias | None) -> x weight^T + bias: few rows without a bias on the
+// kernel of linear.hip, everything else the library's product
+PyObject* linear(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  return guarded(n, 3, [&]() -> PyObject* {
+    Args a{v};
+    const at::Tensor& x = a.tensor(0);
+    const at::Tensor& w = a.tensor(1);
+    need(!watched() && !x._fw_grad(0).defined() && !w._fw_grad(0).defined());
+    if (a.none(2) && x.dim() == 2 && w.dim() == 2 && x.scalar_type() == at::kBFloat16 &&
+        w.scalar_type() == at::kBFloat16 && x.size(1) == w.size(1) && x.stride(1) == 1 &&
+        w.is_contiguous() && x.size(0) <= 64 &&
+        !(at::GradMode::is_enabled() && (x.requires_grad() || w.requires_grad()))) {
+      const int32_t rows = as_i32(x.size(0)), m = as_i32(w.size(0)), k = as_i32(x.size(1));
+      if (nva_linear_preferred(rows, m, k) && x.stride(0) % 8 == 0 && x.stride(0) >= k &&
+          reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+          reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0) {
+        at::Tensor out = empty_bf16({rows, m}, x);
+        void* s = current_stream();
+        launch([&] {
+          return nva_linear(x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), m, rows, m, k, s);
+        });
+        return THPVariable_Wrap(out);
+      }
+    }
+    at::Tensor out;
+    {
+      WithoutGil free;
+      out = a.none(2) ? at::linear(x, w) : at::linear(x, w, a.any(2));
+    }
+    return THPVariable_Wrap(out);
+  });
+}
+
 // (x [T, H, D]) -> its view [T, H * D]
 PyObject* merge_heads(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return guarded(n, 1, [&]() -> PyObject* {
@@ -442,6 +499,7 @@ PyMethodDef methods[] = {
     FAST("paged_attention_varlen", paged_attention_varlen),
     FAST("paged_attention_decode", paged_attention_decode),
     FAST("argmax_rows", argmax_rows),
+    FAST("linear", linear),
     FAST("merge_heads", merge_heads),
     FAST("place", place),
     {nullptr, nullptr, 0, nullptr},
@@ -458,5 +516,11 @@ extern "C" __attribute__((visibility("default"))) PyObject* PyInit__front_end() 
   g_raw_stream = PyObject_GetAttrString(torch_c, "_cuda_getCurrentRawStream");
   Py_DECREF(torch_c);
   if (!g_current_device || !g_raw_stream) return nullptr;
+  PyObject* device_module = PyImport_ImportModule("torch.utils._device");
+  if (!device_module) return nullptr;
+  g_device_context =
+      reinterpret_cast<PyTypeObject*>(PyObject_GetAttrString(device_module, "DeviceContext"));
+  Py_DECREF(device_module);
+  if (!g_device_context) return nullptr;
   return PyModule_Create(&module);
 }

@@ -67,6 +67,8 @@ SIGNATURES = {
                                       _F32, _P, _P, _P, _INT, _I64, _I64, _I64, _I32, _I32, _P,
                                       _P, _P, _P]),
     "nva_silu_mul": (_INT, [_P, _I64, _P, _I64, _I32, _I32, _P]),
+    "nva_linear_preferred": (_INT, [_I32, _I32, _I32]),
+    "nva_linear": (_INT, [_P, _I64, _P, _P, _I64, _I32, _I32, _I32, _P]),
     "nva_verify_metadata": (_INT, [_P, _P, _I32, _P, _I64, _I32, _I32, _P, _P, _P, _P, _I32, _P]),
     "nva_draft_metadata": (_INT, [_P, _P, _P, _I32, _I32, _I32, _P, _I64, _I32, _I32, _I32, _P,
                                   _P, _P, _P]),

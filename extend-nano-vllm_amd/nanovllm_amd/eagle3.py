@@ -14,7 +14,6 @@ from dataclasses import dataclass
 from pathlib import Path
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from nanovllm_amd import kernels as K
@@ -213,7 +212,7 @@ class Eagle3ForCausalLM(nn.Module):
     def sample_greedy(self, hidden_states: torch.Tensor, out: torch.Tensor | None = None):
         """argmax of the draft logits mapped to target ids (eagle3.py:294-296),
         fused in the argmax kernel."""
-        logits = F.linear(hidden_states, self.lm_head.weight)
+        logits = K.linear(hidden_states, self.lm_head.weight)
         return K.argmax_rows(logits, self.d2t, out=out)
 
 

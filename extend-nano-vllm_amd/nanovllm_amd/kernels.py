@@ -691,6 +691,14 @@ def qk_norm_rope_store(qkv: torch.Tensor, positions: torch.Tensor,
     return q
 
 
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """``F.linear``: few bf16 rows without a bias run on the HIP kernel where
+    that is the faster one (``nva_linear_preferred``), the rest on the
+    library."""
+    got = (_front or _front_end()).linear(x, weight, bias)
+    return torch.nn.functional.linear(x, weight, bias) if got is None else got
+
+
 def silu_mul(x: torch.Tensor) -> torch.Tensor:
     """SiluAndMul (layers/activation.py:11-14) on rows [a | b]."""
     got = (_front or _front_end()).silu_mul(x)

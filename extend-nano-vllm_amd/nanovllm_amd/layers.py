@@ -1,8 +1,8 @@
 """Building blocks of the target and draft forwards.
 
-Projection GEMMs stay on torch (hipBLASLt); norms, RoPE, SiLU-and-mul, the
-KV write and the paged attention run in the HIP library.  Module and
-parameter names follow the reference (nanovllm/layers/*.py) so checkpoints
+Projections of few rows run on a HIP kernel, the others stay on torch
+(hipBLASLt); norms, RoPE, SiLU-and-mul, the KV write and the paged attention
+run in the HIP library.  Module and parameter names follow the reference (nanovllm/layers/*.py) so checkpoints
 load unchanged.
 """
 from __future__ import annotations
@@ -48,7 +48,7 @@ class Linear(nn.Module):
         param.data[offset:offset + rows].copy_(loaded)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.weight, self.bias)
+        return K.linear(x, self.weight, self.bias)
 
 
 class Embedding(nn.Module):

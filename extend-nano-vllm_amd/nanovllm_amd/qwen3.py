@@ -9,7 +9,6 @@ the aux-gather kernel only for the rows that need it.
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 from torch import nn
 
 from nanovllm_amd import kernels as K
@@ -98,12 +97,12 @@ class Qwen3ForCausalLM(nn.Module):
                                                          tuple(aux_hidden_state_layers))
 
     def compute_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden_states, self.lm_head.weight)
+        return K.linear(hidden_states, self.lm_head.weight)
 
     def compute_all_logits(self, hidden_states: torch.Tensor) -> torch.Tensor:
         """One logit row per token (the EAGLE3 verify needs every row;
         models/qwen3.py:407-416)."""
-        return F.linear(hidden_states, self.lm_head.weight)
+        return K.linear(hidden_states, self.lm_head.weight)
 
 
 def aux_concat(aux: list[tuple[torch.Tensor, torch.Tensor]],

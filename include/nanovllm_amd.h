@@ -456,6 +456,15 @@ int nva_verify_input_ids(const int32_t *compose, const int32_t *last_tokens, con
 int nva_silu_mul(const void *x, int64_t x_row_stride, void *out, int64_t out_row_stride,
                  int32_t rows, int32_t intermediate, void *stream);
 
+/* out[rows, n] = x[rows, k] . w[n, k]^T in bf16 with fp32 sums: the projections
+ *   of at most 64 rows.  w is contiguous; k must be a multiple of 64, n of 4,
+ *   x_row_stride of 8 and out_row_stride of 4, all pointers 16-byte aligned
+ *   (NVA_ERR_UNSUPPORTED otherwise).  nva_linear_preferred: 1 for the shapes
+ *   where it was measured faster than the library's product. */
+int nva_linear_preferred(int32_t rows, int32_t n, int32_t k);
+int nva_linear(const void *x, int64_t x_row_stride, const void *w, void *out,
+               int64_t out_row_stride, int32_t rows, int32_t n, int32_t k, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -147,6 +147,79 @@ def test_attention_equals_the_python_path(cuda, monkeypatch, fp8, head_major):
         _same(*_both(monkeypatch, decode))
 
 
+LINEAR_SHAPES = [
+    # rows around the 16-row tiles and the limit, K of one chunk, fewer chunks
+    # than waves, a remainder of waves and of depth, N short of a tile
+    (1, 16, 64), (2, 20, 128), (15, 64, 448), (16, 6144, 576), (17, 1024, 1600), (31, 100, 3072),
+    (32, 6148, 256), (33, 4096, 1024), (48, 48, 64), (64, 6160, 2048), (7, 12288, 1024),
+    (9, 12300, 512), (64, 1024, 16384),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", LINEAR_SHAPES)
+def test_linear_rows_against_64_bits(cuda, m, n, k):
+    """nva_linear over every tile shape: half a bf16 ulp of the result (bf16 has 8
+    significant bits: at most 2^-8 of the value, rounded up to 1.01 of it here)
+    plus fp32 sums of K terms, within (K / 32) 2^-24 of the sum of magnitudes
+    (32 products a matrix instruction, chained)."""
+    g = torch.Generator(device=cuda).manual_seed(m + n + k)
+    x = torch.randn(m, k + 8, generator=g, device=cuda).to(BF16)[:, :k]
+    w = (torch.randn(n, k, generator=g, device=cuda) * 0.05).to(BF16)
+    guard = torch.full((m + 1, n + 4), 7.0, dtype=BF16, device=cuda)
+    lib = _native.load()
+    _native.check(lib.nva_linear(x.data_ptr(), x.stride(0), w.data_ptr(), guard.data_ptr(),
+                                 guard.stride(0), m, n, k, K._stream()), "linear")
+    want = x.double() @ w.double().t()
+    bound = want.abs() * 1.01 * 2.0 ** -8 + (x.double().abs() @ w.double().abs().t()) * (k / 32) * 2.0 ** -24
+    assert bool(((guard[:m, :n].double() - want).abs() <= bound + 1e-30).all())
+    assert bool((guard[m:] == 7).all()) and bool((guard[:, n:] == 7).all())   # nothing else written
+    got = K.linear(x, w)
+    assert got.shape == (m, n) and got.is_contiguous()
+    assert bool(((got.double() - want).abs() <= bound + 1e-30).all())
+
+
+@pytest.mark.gpu
+def test_linear_takes_every_form_the_library_takes(cuda):
+    import torch.nn.functional as F
+
+    x, w = torch.randn(5, 128, device=cuda), torch.randn(32, 128, device=cuda)
+    b = torch.randn(32, device=cuda).to(BF16)
+    xb, wb = x.to(BF16), w.to(BF16)
+    assert torch.equal(K.linear(x, w), F.linear(x, w))                       # float32
+    assert torch.equal(K.linear(xb, wb, b), F.linear(xb, wb, b))             # bias
+    three = xb.view(1, 5, 128).expand(2, 5, 128)
+    assert torch.equal(K.linear(three, wb), F.linear(three, wb))
+    odd = torch.randn(32, 129, device=cuda).to(BF16)[:, 1:]
+    assert torch.equal(K.linear(xb, odd), F.linear(xb, odd))                 # strided, misaligned
+    wg = w.clone().requires_grad_()
+    K.linear(x, wg).sum().backward()
+    assert wg.grad is not None
+    wg = wb.clone().requires_grad_()
+    K.linear(xb, wg).sum().backward()
+    assert wg.grad is not None
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert K.linear(xb, wb).dtype == torch.float16
+    tangent = torch.autograd.forward_ad
+    with tangent.dual_level():
+        d = K.linear(tangent.make_dual(xb, xb), wb)
+        assert tangent.unpack_dual(d).tangent is not None
+    rows = torch.vmap(lambda r: K.linear(r, wb))(xb.view(5, 1, 128))
+    assert rows.shape == (5, 1, 32)
+    seen = []
+
+    class Log(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, fn, types, args=(), kwargs=None):
+            seen.append(fn)
+            return fn(*args, **(kwargs or {}))
+
+    with Log():
+        K.linear(xb, wb)
+    assert seen
+    with pytest.raises(RuntimeError):
+        K.linear(xb, wb[:, :64])
+
+
 @pytest.mark.gpu
 def test_other_forms_still_run(cuda):
     """Host lengths, a scale or bound of another number type: the Python path
