@@ -8,7 +8,8 @@
 // 4): every row of a verify step (k+1 positions).  Sequences with more rows
 // than one such tile (prefill) run on the wide-tile kernel below.  Segments
 // come from one of two decompositions:
-//   * stream (single-tile sequences of at most 32 rows over an FP8 cache):
+//   * stream (single-tile sequences of at most 32 rows over an FP8 cache, in
+//     batches of many keys):
 //     per kv head the key chunks of all sequences are laid end to end and
 //     cut into one equal range per SIMD of the device, so every wave streams
 //     the same number of keys whatever the length mix;
@@ -76,7 +77,6 @@ constexpr int kVStage = kChunk * kVPitch;            // dwords of the wave's V s
 constexpr int kSplitKeys = 3072;       // fixed decomposition, one wave per split
 constexpr int kKeysPerSharedWave = 352; // fixed decomposition, several waves per split
 constexpr int kMinSplit = 128;
-constexpr int64_t kMinWaves = 1024;
 // a split spans at most kWave - 2 blocks; blocks hold at least kChunk tokens
 constexpr int kMaxSeqGroups = 8;        // stream mode: up to 8 * 64 sequences
 constexpr int kMinRangeChunks = 4;      // stream mode: at least 128 keys per range
@@ -1719,6 +1719,29 @@ int32_t device_cus() {
   return cus[dev];
 }
 
+// Shared-tile kernel for bf16 64-row tiles: waves per tile and chunks in
+// flight.  NVA_ATTN_TILE=0 selects the one-wave kernel instead; "W,D"
+// (W = 2 or 4, D = 2..4) picks a variant (tuning).
+struct TileChoice {
+  int wpt, depth;
+};
+TileChoice tile_choice() {
+  static const TileChoice c = [] {
+    TileChoice t{4, 4};
+    const char* v = getenv("NVA_ATTN_TILE");
+    if (v) {
+      int w = 0, d = 0;
+      if (atoi(v) == 0) return TileChoice{0, 0};
+      // two waves per tile hold 32 columns' accumulators each: only two
+      // chunks in flight fit their registers without spilling
+      if (sscanf(v, "%d,%d", &w, &d) == 2 && ((w == 2 && d == 2) || (w == 4 && d >= 2 && d <= 4)))
+        t = TileChoice{w, d};
+    }
+    return t;
+  }();
+  return c;
+}
+
 // Split length of the fixed decomposition.  A segment is one (sequence, kv
 // head); `waves` waves share each split.
 //   * Eight waves per split (bf16 tiles of up to 32 rows): 352 keys per
@@ -1742,23 +1765,40 @@ int32_t device_cus() {
 // split, each workgroup's start-up worth ~340 keys of streaming.  With K
 // staged through LDS (two alternating sweeps on one box): 55.2-55.3 at
 // 2816, 55.6-55.7 at 2944, 55.8-55.9 at 2688, 56.5 at 2560 and at 3072,
-// 56.6 at 2432.  The length shrinks in 128-key steps (to a 128-key
-// minimum) only while fewer than kMinWaves waves would be launched, and is
-// capped so that a split spans at most kWave - 2 blocks of block_size tokens
-// (the kernel holds one block id per lane); block_size 0 (unknown: the
-// workspace query) assumes the smallest block, kChunk tokens, which bounds
-// the split count from above.
-void choose_split(int32_t num_seqs, int32_t num_kv_heads, int32_t max_k, int32_t waves,
+// 56.6 at 2432.
+// Fewer segments than the device has places for (a place: a CU for eight-wave
+// segments, half a CU for shared tiles, a SIMD for single waves) take splits
+// of an even share of the longest sequence: about as many segments as places,
+// in one round.  Eight-wave and shared-tile splits round the share count to
+// the nearer (eight waves: two thirds up), since the lengths spread below the
+// longest and a second round costs more than idle CUs (Qwen3-0.6B decode, 24
+// sequences of 300-1000 keys: 17.4 us whole, 22.8 in halves).  Below 256 keys
+// a split gives waves nothing to do, and 32 splits of 128 cost the combine
+// more than they save (4000 keys 13.4 against 12.1), so long sequences stop
+// there, the shortest stay whole (300 keys 8.0 against 8.9 in three), and
+// 64-row tiles over more than 8192 keys stop at 512 (16000: 27.1 against
+// 33.5).  Until about 1024 waves ran at all, lengths used to shrink from the
+// default; measured against that, us per call, one box, alternating:
+//   Qwen3-0.6B decode: 4 x 1000-2000 keys 15.0 -> 13.0, 4 x 4000-8000 33.9 ->
+//   23.2, 8 x 500-1500 20.5 -> 13.5, 12 x 1000-3000 33.4 -> 26.0;
+//   Qwen3-8B verify (6 rows): 4 x 4000-8000 36.8 -> 27.9, 12 x 1000-3000 37.0
+//   -> 25.7; Qwen3-32B verify (8 rows): 1 x 16000 42.8 -> 27.1, 24 x 300-1000
+//   36.4 -> 30.4, 48 x 300-1200 47.7 -> 39.6, FP8 64 x 500-3000 194 -> 115;
+//   slower only 8 x 2000-8000 at 64 rows, 46.0 -> 47.8.
+// The length is capped so that a split spans at most kWave - 2 blocks of
+// block_size tokens (the kernel holds one block id per lane); block_size 0
+// (unknown: the workspace query) assumes the smallest block, kChunk tokens,
+// which bounds the split count from above.
+void choose_split(int32_t num_seqs, int32_t num_kv_heads, int32_t max_k, int32_t waves, bool tile,
                   int32_t block_size, int32_t* split_len, int32_t* max_splits) {
   const int64_t segs = static_cast<int64_t>(num_seqs > 0 ? num_seqs : 1) *
                        (num_kv_heads > 0 ? num_kv_heads : 1);
-  const int64_t base = segs * (waves > 0 ? waves : 1);
   const int32_t mk = max_k > 1 ? max_k : 1;
   const int32_t cus = device_cus();
+  const int32_t whole = (mk + kMinSplit - 1) / kMinSplit * kMinSplit;
   int32_t len;
   if (waves > 1) {
     len = kKeysPerSharedWave * waves;
-    const int32_t whole = (mk + kMinSplit - 1) / kMinSplit * kMinSplit;
     if (segs >= 4 * static_cast<int64_t>(cus) && whole > len) len = whole;
   } else {
     len = kSplitKeys;
@@ -1767,7 +1807,19 @@ void choose_split(int32_t num_seqs, int32_t num_kv_heads, int32_t max_k, int32_t
   }
   const int32_t span = (kWave - 2) * (block_size > 0 ? block_size : kChunk);
   if (len > span) len = span / kMinSplit * kMinSplit;
-  while (len > kMinSplit && base * ((mk + len - 1) / len) < kMinWaves) len -= kMinSplit;
+  const int64_t want = (waves > 1 ? 1 : tile ? 2 : 4) * static_cast<int64_t>(cus);
+  const int64_t parts = waves > 1 ? (3 * want + segs) / (3 * segs)
+                        : tile    ? (2 * want + segs) / (2 * segs)
+                                  : (want + segs - 1) / segs;
+  if (parts > 1) {
+    const int32_t up = waves > 1 || tile ? kMinSplit - 1 : kMinSplit / 2;
+    int32_t even = static_cast<int32_t>(((mk + parts - 1) / parts + up) / kMinSplit * kMinSplit);
+    const int32_t least = waves > 1 ? (mk <= 384 ? whole : mk <= 1024 ? kMinSplit : 2 * kMinSplit)
+                          : tile    ? (mk <= 2048 ? kMinSplit : mk <= 8192 ? 2 * kMinSplit : 4 * kMinSplit)
+                                    : (mk <= 8192 ? kMinSplit : 2 * kMinSplit);
+    if (even < least) even = least;
+    if (even < len) len = even;
+  }
   // NVA_ATTN_SPLIT_KEYS (a multiple of 128) fixes the split length for tuning
   static const int32_t forced = [] {
     const char* v = getenv("NVA_ATTN_SPLIT_KEYS");
@@ -1791,7 +1843,13 @@ void choose_split(int32_t num_seqs, int32_t num_kv_heads, int32_t max_k, int32_t
 //     us, Qwen3-0.6B verify 74.4 -> 65.1 us).  Single tiles of 17-32 rows
 //     at one to two segments per CU run paired mode instead (paired_mode);
 //   * single-tile sequences of up to 32 rows, FP8: stream decomposition with
-//     the chunk loads issued one chunk ahead (502 us against 573 us fixed);
+//     the chunk loads issued one chunk ahead (502 us against 573 us fixed),
+//     where the longest sequences would give each SIMD more than 600 keys
+//     (480 past 4096-key contexts, whose lengths spread more); below that its
+//     prefix scan and its two kernels in a row cost more than the balance
+//     gains: Qwen3-0.6B decode 12 x 300-1000 keys 15.8 us against 12.0 fixed,
+//     1 x 16000 26.6 / 20.9, 24 x 1000-3000 28.1 / 25.5, but 12 x 4000-12000
+//     43 / 57, 8 x 2000-8000 (6 rows) 33.2 / 35.0;
 //   * bf16 64-row tiles: the shared-tile kernel, four waves per tile with
 //     every chunk loaded once per workgroup and four chunks in flight
 //     (Qwen3-32B verify, config 5's shapes: 425-428 us against 477 us for
@@ -1810,11 +1868,14 @@ int env_choice(const char* name) {
   return v ? (atoi(v) != 0) : -1;
 }
 
-bool stream_mode(int32_t num_seqs, int32_t max_q, int32_t qtile, int32_t group, bool fp8) {
+bool stream_mode(int32_t num_seqs, int32_t hkv, int32_t max_q, int32_t max_k, int32_t qtile,
+                 int32_t group, bool fp8) {
   static const int forced = env_choice("NVA_ATTN_STREAM");
   if (forced == 0 || max_q > qtile || num_seqs > kMaxSeqGroups * kWave) return false;
   if (forced == 1) return max_q * group <= (fp8 ? 32 : 16);
-  return fp8 && max_q * group <= 32;
+  if (!fp8 || max_q * group > 32) return false;
+  return static_cast<int64_t>(num_seqs) * hkv * max_k >
+         (max_k <= 4096 ? 600 : 480) * static_cast<int64_t>(4 * device_cus());
 }
 
 bool pipelined(int nt, bool fp8) {
@@ -1946,8 +2007,8 @@ size_t workspace_bytes(int32_t num_seqs, int32_t num_tokens, int32_t hq, int32_t
   const int32_t qtile = choose_qtile(max_q, hkv > 0 ? hq / hkv : 1);
   const int32_t group = hkv > 0 ? hq / hkv : 1;
   size_t bytes = 0;
-  if (stream_mode(num_seqs, max_q, qtile, group, false) ||
-      stream_mode(num_seqs, max_q, qtile, group, true)) {
+  if (stream_mode(num_seqs, hkv, max_q, max_k, qtile, group, false) ||
+      stream_mode(num_seqs, hkv, max_q, max_k, qtile, group, true)) {
     bytes = partials_bytes(num_tokens, hq, stream_max_splits(max_k));
   }
   const int32_t n_qtiles = (max_q + qtile - 1) / qtile;
@@ -1959,37 +2020,14 @@ size_t workspace_bytes(int32_t num_seqs, int32_t num_tokens, int32_t hq, int32_t
   const int nt = tile_mfmas(qtile * (hkv > 0 ? hq / hkv : 1));
   // either KV dtype: the larger split count of the two wave choices
   int32_t len, ms, ms_fp8;
-  choose_split(num_seqs, hkv, max_k, segment_waves(nt, false), 0, &len, &ms);
-  choose_split(num_seqs, hkv, max_k, segment_waves(nt, true), 0, &len, &ms_fp8);
+  choose_split(num_seqs, hkv, max_k, segment_waves(nt, false), tile_choice().wpt && nt >= 4, 0, &len, &ms);
+  choose_split(num_seqs, hkv, max_k, segment_waves(nt, true), false, 0, &len, &ms_fp8);
   ms = ms_fp8 > ms ? ms_fp8 : ms;
   if (ms > 1) {
     const size_t fixed = partials_bytes(num_tokens, hq, ms);
     bytes = fixed > bytes ? fixed : bytes;
   }
   return bytes;
-}
-
-// Shared-tile kernel for bf16 64-row tiles: waves per tile and chunks in
-// flight.  NVA_ATTN_TILE=0 selects the one-wave kernel instead; "W,D"
-// (W = 2 or 4, D = 2..4) picks a variant (tuning).
-struct TileChoice {
-  int wpt, depth;
-};
-TileChoice tile_choice() {
-  static const TileChoice c = [] {
-    TileChoice t{4, 4};
-    const char* v = getenv("NVA_ATTN_TILE");
-    if (v) {
-      int w = 0, d = 0;
-      if (atoi(v) == 0) return TileChoice{0, 0};
-      // two waves per tile hold 32 columns' accumulators each: only two
-      // chunks in flight fit their registers without spilling
-      if (sscanf(v, "%d,%d", &w, &d) == 2 && ((w == 2 && d == 2) || (w == 4 && d >= 2 && d <= 4)))
-        t = TileChoice{w, d};
-    }
-    return t;
-  }();
-  return c;
 }
 
 template <int WPT>
@@ -2098,7 +2136,7 @@ int run_attention(AttnParams& p, int kv_dtype, void* workspace, size_t workspace
     return NVA_ERR_UNSUPPORTED;
   const bool fp8 = kv_dtype == NVA_KV_FP8_E4M3;
   const bool wide = p.n_qtiles > 1;
-  const bool stream = stream_mode(p.num_seqs, p.max_q, p.qtile, p.group, fp8);
+  const bool stream = stream_mode(p.num_seqs, p.hkv, p.max_q, p.max_k, p.qtile, p.group, fp8);
   const int nt = tile_mfmas(tile_rows);
   // paired mode's whole-sequence split must fit the kernel's block ids
   const int32_t mk = p.max_k > 1 ? p.max_k : 1;
@@ -2133,7 +2171,7 @@ int run_attention(AttnParams& p, int kv_dtype, void* workspace, size_t workspace
     p.pair_rows = device_cus() / p.hkv;
     grid = dim3(p.hkv, p.num_seqs, 1);
   } else {
-    choose_split(p.num_seqs, p.hkv, p.max_k, wps, p.block_size, &p.split_len,
+    choose_split(p.num_seqs, p.hkv, p.max_k, wps, !fp8 && nt >= 4 && tile_choice().wpt, p.block_size, &p.split_len,
                  &p.max_splits);
     // the kernel keeps one block id per lane: a split may touch at most kWave blocks
     if (p.split_len / p.block_size + 2 > kWave) return NVA_ERR_UNSUPPORTED;

@@ -1208,3 +1208,34 @@ def test_several_query_tiles_skip_invalid_blocks_and_scale(K, cuda, fp8):
                                  np.array([n], np.int32), sub.numpy(), 128 ** -0.5, ks, vs)
     err = np.abs(out.float().cpu().numpy() - ref).max()
     assert err <= ATTN_TOL, err
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hq,q_len", [(8, [1, 1, 0, 1, 1]), (32, [6, 3, 1, 6, 2]), (64, [8, 8, 5, 8, 0])])
+def test_small_batch_decompositions(K, cuda, hq, q_len, fp8):
+    """One batch under bounds that give every split choice of a small batch
+    (whole, a few even shares, the 128-, 256- and 512-key minima; over FP8
+    also the stream decomposition): all equal to the oracle."""
+    case = paged_case(seed=31, batch=5, q_len=q_len, ctx_lo=1, ctx_hi=1500, hq=hq, hkv=8,
+                      block_size=256)
+    kc, vc = case["k_cache"], case["v_cache"]
+    if fp8:
+        kc, vc = kc.float().to(torch.float8_e4m3fn), vc.float().to(torch.float8_e4m3fn)
+    ref = oracle.paged_attention(bits(case["q"]), bits(kc), bits(vc), case["cu_q"].numpy(),
+                                 case["lens"].numpy(), case["block_tables"].numpy(), 128 ** -0.5)
+    args = [case["q"].to(cuda), kc.to(cuda), vc.to(cuda), case["cu_q"].to(cuda), case["cu_k"].to(cuda)]
+    longest = int(case["lens"].max())
+    for bound in (longest, 1800, 2100, 4200, 9000, 20000, 40000):
+        out = K.paged_attention_varlen(*args, max(q_len), bound, 128 ** -0.5,
+                                       case["block_tables"].to(cuda))
+        torch.cuda.synchronize()
+        err = np.abs(out.float().cpu().numpy() - ref).max()
+        assert err <= ATTN_TOL, (bound, err)
+    short = [min(int(n), 380) for n in case["lens"]]    # whole sequences below the split minimum
+    cu_k = torch.tensor([0] + np.cumsum(short).tolist(), dtype=torch.int32, device=cuda)
+    ref = oracle.paged_attention(bits(case["q"]), bits(kc), bits(vc), case["cu_q"].numpy(),
+                                 np.array(short, np.int32), case["block_tables"].numpy(), 128 ** -0.5)
+    out = K.paged_attention_varlen(*args[:4], cu_k, max(q_len), 380, 128 ** -0.5,
+                                   case["block_tables"].to(cuda))
+    err = np.abs(out.float().cpu().numpy() - ref).max()
+    assert err <= ATTN_TOL, err
