@@ -108,6 +108,10 @@ typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void store_streamed(uint16_t* p, uint16_t v) {
   __builtin_nontemporal_store(v, p);
 }
+typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void store_streamed(uint2* p, uint2 v) {
+  __builtin_nontemporal_store(__builtin_bit_cast(u32x2_t, v), reinterpret_cast<u32x2_t*>(p));
+}
 __device__ __forceinline__ void store_streamed(uint4* p, uint4 v) {
   __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, v), reinterpret_cast<u32x4_t*>(p));
 }

@@ -24,12 +24,6 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return s;
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int m = kWave / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, kWave);
-  return v;
-}
-
 // RMSNorm of one row, optionally after adding a residual row:
 //   s = f32(x) (+ f32(residual));  residual_out = bf16(s)
 //   out = bf16( bf16(s * rsqrt(mean(s^2) + eps)) * weight )
@@ -180,128 +174,195 @@ rms_norm_kernel(const uint16_t* __restrict__ x, int64_t x_stride,
   }
 }
 
-// Per-head RMSNorm (optional) + neox rotary embedding for the q and k heads
-// of a fused QKV row; one wave per head, lane l owns elements l and l + 64
-// (the two halves the rotation pairs).
+// Per-head RMSNorm (optional) + neox rotary embedding for the q and k heads of
+// a fused QKV row, and (STORE) the write of the rotated keys and of the value
+// heads to the paged cache in the same launch:
 //   norm:  x = bf16(bf16(x * rsqrt(mean(x^2) + eps)) * w)   (qwen3.py:87-96)
 //   rope:  y1 = x1*cos - x2*sin, y2 = x2*cos + x1*sin in fp32, rounded to bf16
 //          with cos/sin = cos_sin[pos][i], cos_sin[pos][64 + i]
 //          (rotary_embedding.py:6-48)
-__global__ void __launch_bounds__(kNormThreads)
-qk_norm_rope_kernel(const uint16_t* __restrict__ qkv, int64_t row_stride,
-                    const int64_t* __restrict__ positions, const uint16_t* __restrict__ q_w,
-                    const uint16_t* __restrict__ k_w, const float* __restrict__ cos_sin,
-                    int32_t max_pos, int32_t num_tokens, int32_t hq, int32_t hkv, float eps,
-                    uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_out) {
-  const int t = blockIdx.y;
-  const int head = blockIdx.x * (kNormThreads / kWave) + threadIdx.x / kWave;
-  const int lane = wave_lane();
-  if (t >= num_tokens || head >= hq + hkv) return;
-  const bool is_q = head < hq;
-  const uint16_t* src = qkv + static_cast<int64_t>(t) * row_stride + static_cast<int64_t>(head) * 128;
-  // every load is issued before the first use (the position's cos/sin row
-  // behind the position itself, both ahead of the norm's reduction)
-  int64_t pos = positions[t];
-  float x1 = bf16_to_f32(src[lane]);
-  float x2 = bf16_to_f32(src[lane + 64]);
-  const uint16_t* w = is_q ? q_w : k_w;
-  const float w1 = w ? bf16_to_f32(w[lane]) : 1.0f;
-  const float w2 = w ? bf16_to_f32(w[lane + 64]) : 1.0f;
-  pos = pos < 0 ? 0 : (pos >= max_pos ? max_pos - 1 : pos);
-  const float c = cos_sin[pos * 128 + lane];
-  const float s = cos_sin[pos * 128 + 64 + lane];
-  if (w) {
-    const float inv = rsqrtf(wave_sum(x1 * x1 + x2 * x2) / 128.0f + eps);
-    x1 = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(x1 * inv)) * w1));
-    x2 = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(x2 * inv)) * w2));
-  }
-  const float y1 = x1 * c - x2 * s;
-  const float y2 = x2 * c + x1 * s;
-  uint16_t* dst = is_q ? q_out + (static_cast<int64_t>(t) * hq + head) * 128
-                       : k_out + (static_cast<int64_t>(t) * hkv + (head - hq)) * 128;
-  dst[lane] = f32_to_bf16(y1);
-  dst[lane + 64] = f32_to_bf16(y2);
-}
+// Heads [0, hq) are queries (to q_out), [hq, hq + hkv) keys (to k_out, or
+// rounded to bf16 and then to the cache at the token's slot, e4m3(bf16 /
+// k_scale) for FP8), [hq + hkv, hq + 2 hkv) values (copied to the cache, e4m3(
+// bf16 / v_scale) for FP8); a slot that is negative or past the cache is
+// skipped.  Every value written is the one store_kvcache would write.
+//
+// Memory bound at prefill sizes, latency bound below.  16 lanes take a head:
+// lane i the elements 4 i .. 4 i + 3 and 64 + 4 i .. (the two halves the
+// rotation pairs) as 8-byte loads and stores, four heads a wave.  With a head
+// a wave and 2-byte accesses, 384 tokens of 48 heads took 7.7 us, 1024 of 32
+// heads 12.2, 16384 of 48 heads 177 (2.3 TB/s); now 5.1, 6.0 and 72.6 (5.5).
+enum class KeyTo { kTensor, kCacheBf16, kCacheFp8 };
 
-// qk_norm_rope_kernel and store_kvcache in one launch: waves [0, hq) take
-// the query heads (normalised, rotated, written to q_out), waves [hq, hq +
-// hkv) the key heads (normalised, rotated, rounded to bf16, then written to
-// the paged cache at the token's slot, e4m3(bf16 / k_scale) for FP8) and
-// waves [hq + hkv, hq + 2 hkv) the value heads (copied to the cache, e4m3(
-// bf16 / v_scale) for FP8).  Every value written is the one the two separate
-// kernels write; a slot that is negative or past the cache is skipped.
 struct SlotPages {
   int64_t blk_stride, tok_stride, head_stride;  // elements
   int32_t block_size;
   int64_t num_slots;
 };
 
-template <bool FP8>
-__device__ __forceinline__ void put_cache_pair(void* cache, int64_t dst, int lane, uint16_t a,
-                                               uint16_t b, float scale) {
-  if constexpr (FP8) {
-    uint8_t* c = static_cast<uint8_t*>(cache) + dst;
-    c[lane] = static_cast<uint8_t>(f32_to_e4m3(bf16_to_f32(a) / scale));
-    c[lane + 64] = static_cast<uint8_t>(f32_to_e4m3(bf16_to_f32(b) / scale));
+// The sum of p over the 64 element pairs of a head, in the order of a 64-lane
+// butterfly (32, 16, 8, 4, 2, 1) over pairs 4 i + e: a row rotation by n takes
+// the place of the exchange with lane i ^ n, since the sums so far repeat
+// every 2 n lanes.
+template <int N>
+__device__ __forceinline__ float row_ror_add(float v) {
+  const int r = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + N, 0xF, 0xF, false);
+  return v + __builtin_bit_cast(float, r);
+}
+__device__ __forceinline__ float head_sum(float (&p)[4]) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    p[e] = row_ror_add<1>(row_ror_add<2>(row_ror_add<4>(row_ror_add<8>(p[e]))));
+  return (p[0] + p[2]) + (p[1] + p[3]);
+}
+
+template <bool VEC>
+__device__ __forceinline__ void load4(const uint16_t* p, float (&v)[4]) {
+  if constexpr (VEC) {
+    const uint2 w = *reinterpret_cast<const uint2*>(p);
+    v[0] = bf16_to_f32(w.x & 0xFFFFu);
+    v[1] = bf16_to_f32(w.x >> 16);
+    v[2] = bf16_to_f32(w.y & 0xFFFFu);
+    v[3] = bf16_to_f32(w.y >> 16);
   } else {
-    // one full 128-byte line per instruction (64 lanes x 2 bytes)
-    uint16_t* c = static_cast<uint16_t*>(cache) + dst;
-    store_streamed(c + lane, a);
-    store_streamed(c + lane + 64, b);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = bf16_to_f32(p[e]);
+  }
+}
+template <bool VEC>
+__device__ __forceinline__ void load4(const float* p, float (&v)[4]) {
+  if constexpr (VEC) {
+    const float4 w = *reinterpret_cast<const float4*>(p);
+    v[0] = w.x; v[1] = w.y; v[2] = w.z; v[3] = w.w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = p[e];
+  }
+}
+template <bool VEC>
+__device__ __forceinline__ void put4(uint16_t* p, const uint16_t (&v)[4]) {
+  if constexpr (VEC) {
+    store_streamed(reinterpret_cast<uint2*>(p),
+                   make_uint2(v[0] | (static_cast<uint32_t>(v[1]) << 16),
+                              v[2] | (static_cast<uint32_t>(v[3]) << 16)));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) store_streamed(p + e, v[e]);
+  }
+}
+// f32_to_e4m3 of two values in the low half of the result, by gfx950's
+// conversion (round to nearest even, subnormals included).  What is too large,
+// where f32_to_e4m3 saturates, it makes NaN, and NaN loses its sign.  Eight of
+// the software conversions in a lane cost ~1 us a launch.
+__device__ __forceinline__ uint32_t e4m3_pair(float a, float b) {
+  const uint32_t w = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(
+      __builtin_amdgcn_fmed3f(a, -448.0f, 448.0f), __builtin_amdgcn_fmed3f(b, -448.0f, 448.0f), 0, false));
+  auto pick = [](float x, uint32_t byte) {
+    return x != x ? ((__float_as_uint(x) >> 24) & 0x80u) | 0x7Fu : byte;
+  };
+  return pick(a, w & 0xFFu) | (pick(b, (w >> 8) & 0xFFu) << 8);
+}
+template <bool VEC>
+__device__ __forceinline__ void put4_e4m3(uint8_t* p, const uint16_t (&v)[4], float scale) {
+  float x[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = bf16_to_f32(v[e]) / scale;
+  const uint32_t w = e4m3_pair(x[0], x[1]) | (e4m3_pair(x[2], x[3]) << 16);
+  if constexpr (VEC) {
+    *reinterpret_cast<uint32_t*>(p) = w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p[e] = static_cast<uint8_t>(w >> (8 * e));
   }
 }
 
-template <bool FP8>
+template <KeyTo TO, bool VEC>
 __global__ void __launch_bounds__(kNormThreads)
-qk_norm_rope_store_kernel(const uint16_t* __restrict__ qkv, int64_t row_stride,
-                          const int64_t* __restrict__ positions, const uint16_t* __restrict__ q_w,
-                          const uint16_t* __restrict__ k_w, const float* __restrict__ cos_sin,
-                          int32_t max_pos, int32_t num_tokens, int32_t hq, int32_t hkv, float eps,
-                          uint16_t* __restrict__ q_out, void* __restrict__ k_cache,
-                          void* __restrict__ v_cache, SlotPages pages,
-                          const int32_t* __restrict__ slot_mapping,
-                          const float* __restrict__ k_scale_p, const float* __restrict__ v_scale_p) {
+qk_norm_rope_kernel(const uint16_t* __restrict__ qkv, int64_t row_stride,
+                    const int64_t* __restrict__ positions, const uint16_t* __restrict__ q_w,
+                    const uint16_t* __restrict__ k_w, const float* __restrict__ cos_sin,
+                    int32_t max_pos, int32_t hq, int32_t hkv, float eps,
+                    uint16_t* __restrict__ q_out, void* __restrict__ k_out,
+                    void* __restrict__ v_cache, SlotPages pages,
+                    const int32_t* __restrict__ slot_mapping,
+                    const float* __restrict__ k_scale_p, const float* __restrict__ v_scale_p) {
+  constexpr bool STORE = TO != KeyTo::kTensor;
   const int t = blockIdx.y;
-  const int head = blockIdx.x * (kNormThreads / kWave) + threadIdx.x / kWave;
-  const int lane = wave_lane();
-  if (t >= num_tokens || head >= hq + 2 * hkv) return;
-  const uint16_t* src = qkv + static_cast<int64_t>(t) * row_stride + static_cast<int64_t>(head) * 128;
+  const int head = blockIdx.x * (kNormThreads / 16) + threadIdx.x / 16;
+  const int d0 = 4 * (threadIdx.x & 15);
+  if (head >= hq + (STORE ? 2 : 1) * hkv) return;
+  const uint16_t* src = qkv + static_cast<int64_t>(t) * row_stride + static_cast<int64_t>(head) * 128 + d0;
   int64_t dst = 0;
-  if (head >= hq) {
+  if (STORE && head >= hq) {
     const int64_t slot = slot_mapping[t];
     if (slot < 0 || slot >= pages.num_slots) return;
-    const int kvh = (head - hq) % hkv;
     dst = (slot / pages.block_size) * pages.blk_stride + (slot % pages.block_size) * pages.tok_stride +
-          kvh * pages.head_stride;
+          ((head - hq) % hkv) * pages.head_stride + d0;
   }
-  if (head >= hq + hkv) {
-    put_cache_pair<FP8>(v_cache, dst, lane, src[lane], src[lane + 64],
-                        FP8 && v_scale_p ? *v_scale_p : 1.0f);
+  // every load is issued before the first use (the position's cos/sin row
+  // behind the position itself, both ahead of the norm's reduction)
+  int64_t pos = positions[t];
+  float x1[4], x2[4];
+  load4<VEC>(src, x1);
+  load4<VEC>(src + 64, x2);
+  uint16_t y1[4], y2[4];
+  if (STORE && head >= hq + hkv) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {   // the bits as they were
+      y1[e] = static_cast<uint16_t>(__float_as_uint(x1[e]) >> 16);
+      y2[e] = static_cast<uint16_t>(__float_as_uint(x2[e]) >> 16);
+    }
+    if constexpr (TO == KeyTo::kCacheFp8) {
+      const float scale = v_scale_p ? *v_scale_p : 1.0f;
+      put4_e4m3<VEC>(static_cast<uint8_t*>(v_cache) + dst, y1, scale);
+      put4_e4m3<VEC>(static_cast<uint8_t*>(v_cache) + dst + 64, y2, scale);
+    } else {
+      put4<VEC>(static_cast<uint16_t*>(v_cache) + dst, y1);
+      put4<VEC>(static_cast<uint16_t*>(v_cache) + dst + 64, y2);
+    }
     return;
   }
   const bool is_q = head < hq;
-  int64_t pos = positions[t];
-  float x1 = bf16_to_f32(src[lane]);
-  float x2 = bf16_to_f32(src[lane + 64]);
   const uint16_t* w = is_q ? q_w : k_w;
-  const float w1 = w ? bf16_to_f32(w[lane]) : 1.0f;
-  const float w2 = w ? bf16_to_f32(w[lane + 64]) : 1.0f;
-  pos = pos < 0 ? 0 : (pos >= max_pos ? max_pos - 1 : pos);
-  const float c = cos_sin[pos * 128 + lane];
-  const float s = cos_sin[pos * 128 + 64 + lane];
+  float w1[4], w2[4], c[4], s[4];
   if (w) {
-    const float inv = rsqrtf(wave_sum(x1 * x1 + x2 * x2) / 128.0f + eps);
-    x1 = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(x1 * inv)) * w1));
-    x2 = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(x2 * inv)) * w2));
+    load4<VEC>(w + d0, w1);
+    load4<VEC>(w + d0 + 64, w2);
   }
-  const uint16_t y1 = f32_to_bf16(x1 * c - x2 * s);
-  const uint16_t y2 = f32_to_bf16(x2 * c + x1 * s);
+  pos = pos < 0 ? 0 : (pos >= max_pos ? max_pos - 1 : pos);
+  load4<VEC>(cos_sin + pos * 128 + d0, c);
+  load4<VEC>(cos_sin + pos * 128 + 64 + d0, s);
+  if (w) {
+    float p[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p[e] = x1[e] * x1[e] + x2[e] * x2[e];
+    const float inv = rsqrtf(head_sum(p) / 128.0f + eps);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x1[e] = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(x1[e] * inv)) * w1[e]));
+      x2[e] = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(x2[e] * inv)) * w2[e]));
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    y1[e] = f32_to_bf16(x1[e] * c[e] - x2[e] * s[e]);
+    y2[e] = f32_to_bf16(x2[e] * c[e] + x1[e] * s[e]);
+  }
   if (is_q) {
-    uint16_t* qd = q_out + (static_cast<int64_t>(t) * hq + head) * 128;
-    store_streamed(qd + lane, y1);
-    store_streamed(qd + lane + 64, y2);
+    uint16_t* q = q_out + (static_cast<int64_t>(t) * hq + head) * 128 + d0;
+    put4<VEC>(q, y1);
+    put4<VEC>(q + 64, y2);
+  } else if constexpr (TO == KeyTo::kTensor) {
+    uint16_t* k = static_cast<uint16_t*>(k_out) + (static_cast<int64_t>(t) * hkv + (head - hq)) * 128 + d0;
+    put4<VEC>(k, y1);
+    put4<VEC>(k + 64, y2);
+  } else if constexpr (TO == KeyTo::kCacheFp8) {
+    const float scale = k_scale_p ? *k_scale_p : 1.0f;
+    put4_e4m3<VEC>(static_cast<uint8_t*>(k_out) + dst, y1, scale);
+    put4_e4m3<VEC>(static_cast<uint8_t*>(k_out) + dst + 64, y2, scale);
   } else {
-    put_cache_pair<FP8>(k_cache, dst, lane, y1, y2, FP8 && k_scale_p ? *k_scale_p : 1.0f);
+    put4<VEC>(static_cast<uint16_t*>(k_out) + dst, y1);
+    put4<VEC>(static_cast<uint16_t*>(k_out) + dst + 64, y2);
   }
 }
 
@@ -412,6 +473,18 @@ extern "C" int nva_add_then_rms_norm(const void* x, int64_t x_row_stride, const 
                                    stream);
 }
 
+namespace {
+
+bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
+
+// the 8- and 16-byte accesses of qk_norm_rope_kernel's inputs
+bool rows_aligned(const void* qkv, int64_t row_stride, const void* q_w, const void* k_w,
+                  const void* cos_sin) {
+  return aligned8(qkv) && row_stride % 4 == 0 && aligned8(q_w) && aligned8(k_w) && aligned16(cos_sin);
+}
+
+}  // namespace
+
 extern "C" int nva_qk_norm_rope(const void* qkv, int64_t row_stride, const int64_t* positions,
                                 const void* q_norm_weight, const void* k_norm_weight,
                                 const float* cos_sin, int32_t max_position, int32_t num_tokens,
@@ -425,13 +498,16 @@ extern "C" int nva_qk_norm_rope(const void* qkv, int64_t row_stride, const int64
       row_stride < static_cast<int64_t>(num_q_heads + num_kv_heads) * head_dim)
     return NVA_ERR_ARG;
   if ((q_norm_weight == nullptr) != (k_norm_weight == nullptr)) return NVA_ERR_ARG;
-  const int heads_per_block = kNormThreads / kWave;
+  const int heads_per_block = kNormThreads / 16;
   dim3 grid((num_q_heads + num_kv_heads + heads_per_block - 1) / heads_per_block, num_tokens);
-  qk_norm_rope_kernel<<<grid, kNormThreads, 0, static_cast<hipStream_t>(stream)>>>(
+  const bool vec = rows_aligned(qkv, row_stride, q_norm_weight, k_norm_weight, cos_sin) &&
+                   aligned8(q_out) && aligned8(k_out);
+  auto* kern = vec ? qk_norm_rope_kernel<KeyTo::kTensor, true> : qk_norm_rope_kernel<KeyTo::kTensor, false>;
+  kern<<<grid, kNormThreads, 0, static_cast<hipStream_t>(stream)>>>(
       static_cast<const uint16_t*>(qkv), row_stride, positions,
       static_cast<const uint16_t*>(q_norm_weight), static_cast<const uint16_t*>(k_norm_weight),
-      cos_sin, max_position, num_tokens, num_q_heads, num_kv_heads, eps,
-      static_cast<uint16_t*>(q_out), static_cast<uint16_t*>(k_out));
+      cos_sin, max_position, num_q_heads, num_kv_heads, eps, static_cast<uint16_t*>(q_out), k_out,
+      nullptr, SlotPages{}, nullptr, nullptr, nullptr);
   return launch_status();
 }
 
@@ -455,15 +531,22 @@ extern "C" int nva_qk_norm_rope_store(
   if ((q_norm_weight == nullptr) != (k_norm_weight == nullptr)) return NVA_ERR_ARG;
   const SlotPages pages{cache_block_stride, cache_token_stride, cache_head_stride, block_size,
                         static_cast<int64_t>(num_blocks) * block_size};
-  const int heads_per_block = kNormThreads / kWave;
+  const int heads_per_block = kNormThreads / 16;
   dim3 grid((num_q_heads + 2 * num_kv_heads + heads_per_block - 1) / heads_per_block, num_tokens);
-  auto* kern = kv_dtype == NVA_KV_BF16 ? qk_norm_rope_store_kernel<false>
-                                       : qk_norm_rope_store_kernel<true>;
+  const bool vec = rows_aligned(qkv, row_stride, q_norm_weight, k_norm_weight, cos_sin) &&
+                   aligned8(q_out) && aligned8(k_cache) && aligned8(v_cache) &&
+                   cache_block_stride % 4 == 0 && cache_token_stride % 4 == 0 &&
+                   cache_head_stride % 4 == 0;
+  auto* kern = kv_dtype == NVA_KV_BF16
+                   ? (vec ? qk_norm_rope_kernel<KeyTo::kCacheBf16, true>
+                          : qk_norm_rope_kernel<KeyTo::kCacheBf16, false>)
+                   : (vec ? qk_norm_rope_kernel<KeyTo::kCacheFp8, true>
+                          : qk_norm_rope_kernel<KeyTo::kCacheFp8, false>);
   kern<<<grid, kNormThreads, 0, static_cast<hipStream_t>(stream)>>>(
       static_cast<const uint16_t*>(qkv), row_stride, positions,
       static_cast<const uint16_t*>(q_norm_weight), static_cast<const uint16_t*>(k_norm_weight),
-      cos_sin, max_position, num_tokens, num_q_heads, num_kv_heads, eps,
-      static_cast<uint16_t*>(q_out), k_cache, v_cache, pages, slot_mapping, k_scale, v_scale);
+      cos_sin, max_position, num_q_heads, num_kv_heads, eps, static_cast<uint16_t*>(q_out), k_cache,
+      v_cache, pages, slot_mapping, k_scale, v_scale);
   return launch_status();
 }
 

@@ -1239,3 +1239,25 @@ def test_small_batch_decompositions(K, cuda, hq, q_len, fp8):
                                    case["block_tables"].to(cuda))
     err = np.abs(out.float().cpu().numpy() - ref).max()
     assert err <= ATTN_TOL, err
+
+
+@pytest.mark.parametrize("scale", [1.0, 0.75, 3e-5])
+def test_fp8_store_of_every_bf16_value_equals_store_kvcache(K, cuda, scale):
+    """The fused launch's FP8 conversion against store_kvcache's (oracle-tested)
+    over all bf16 bit patterns: subnormals, ties, saturation, infinities, NaN;
+    aligned rows and rows one element off (the element path)."""
+    v = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).view(64, 8, 128)
+    for off in (0, 1):
+        rows = torch.zeros(64, 1 + 24 * 128, dtype=torch.bfloat16)
+        qkv = rows[:, off:off + 24 * 128]
+        qkv[:, 16 * 128:] = v.view(64, -1)
+        qkv = rows.to(cuda)[:, off:off + 24 * 128] if off else qkv.contiguous().to(cuda)
+        pos = torch.zeros(64, dtype=torch.int64, device=cuda)
+        slots = torch.arange(64, dtype=torch.int32, device=cuda)
+        cos = torch.ones(1, 128, device=cuda)
+        a = torch.zeros(4, 1, 256, 8, 128, device=cuda).to(torch.float8_e4m3fn)
+        sc = torch.tensor([scale], device=cuda)
+        K.qk_norm_rope_store(qkv, pos, None, None, cos, 8, 8, 128, 1e-6, a[0], a[1], slots, sc, sc)
+        K.store_kvcache(torch.zeros(64, 8, 128, dtype=torch.bfloat16, device=cuda),
+                        v.to(cuda), a[2], a[3], slots, sc, sc)
+        np.testing.assert_array_equal(bits(a[1].cpu()), bits(a[3].cpu()))
