@@ -506,7 +506,12 @@ class ModelRunner:
             raise IndexError("a draft position has no page in its block table")
         ids = bt[np.arange(b)[None, :], np.minimum(blk, bt.shape[1] - 1)].astype(np.int64)
         slots = np.where(need, ids * self.block_size + pos % self.block_size, -1).astype(np.int32)
-        return pos, slots, (pos + 1).astype(np.int32)
+        # steps past the last one see the keys written so far: their own slot
+        # may never have been written, and its page's old contents would decide
+        # their tokens
+        written = lens - 1 + np.maximum(np.asarray(limits, dtype=np.int64) - 1, 0)
+        ctx = np.maximum(np.minimum(pos + 1, written[None, :]), 1)
+        return pos, slots, ctx.astype(np.int32)
 
     def _use_graphs(self) -> bool:
         return not self.enforce_eager

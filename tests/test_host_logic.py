@@ -559,3 +559,20 @@ def test_lookahead_churn_leaves_cached_prefix_pages_alone():
     hits = bm.stats["prefix_cache_hits"]
     bm.allocate(c)
     assert bm.stats["prefix_cache_hits"] == hits + 2 and c.block_table == keyed
+
+
+def test_draft_steps_past_the_last_proposal_see_written_keys_only():
+    """A sequence with one proposal left writes no draft K/V, one with three
+    writes two positions; the later steps' contexts stop there, so their
+    (discarded) tokens do not depend on what a page held before."""
+    from nanovllm_amd.engine import model_runner as mr
+
+    runner = mr.ModelRunner.__new__(mr.ModelRunner)
+    runner.block_size = 256
+    seqs = [Sequence(list(range(n))) for n in (100, 255, 40)]
+    for i, seq in enumerate(seqs):
+        seq.block_table = [2 * i, 2 * i + 1]
+    _, slots, ctx = runner._draft_step_metadata(seqs, [1, 3, 5], 5)
+    assert ctx[:, 0].tolist() == [99, 99, 99, 99] and set(slots[:, 0].tolist()) == {-1}
+    assert ctx[:, 1].tolist() == [255, 256, 256, 256] and slots[2:, 1].tolist() == [-1, -1]
+    assert ctx[:, 2].tolist() == [40, 41, 42, 43] and min(slots[:, 2].tolist()) >= 0
