@@ -125,6 +125,7 @@ def load_front_end():
     """The CPython module in front of the library (csrc/front_end.cpp)."""
     global _front
     if _front is None:
+        import torch  # noqa: F401  - the module links against torch's libraries
         load()
         if not os.path.exists(FRONT_PATH):
             raise NativeLibraryError(f"{FRONT_PATH} is missing: build it with `make -C {CSRC_DIR}` "

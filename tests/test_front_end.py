@@ -1,5 +1,9 @@
 """The native front end against the Python path behind it: bit-equal results
 for every form both take, and hands off (None) everything else."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -235,3 +239,11 @@ def test_other_forms_still_run(cuda):
         assert torch.equal(K.paged_attention_decode(q, kv[0], kv[1], n, table, s, b), want)
     with pytest.raises(ValueError):
         K.paged_attention_decode(q, kv[0], kv[1], lens.tolist(), table, 0.5, 16)
+
+
+def test_loads_in_a_process_that_has_not_imported_torch():
+    """As a build check does: the module's own libraries include torch's."""
+    code = "from nanovllm_amd import _native; _native.load_front_end()"
+    pkg = os.path.dirname(os.path.dirname(os.path.abspath(_native.__file__)))
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=300,
+                   env={**os.environ, "PYTHONPATH": pkg})
