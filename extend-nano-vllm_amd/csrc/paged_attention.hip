@@ -1868,14 +1868,19 @@ int env_choice(const char* name) {
   return v ? (atoi(v) != 0) : -1;
 }
 
+// What the stream decomposition takes (and, bf16, only when it is forced).
+bool stream_takes(int32_t num_seqs, int32_t max_q, int32_t qtile, int32_t group, bool fp8) {
+  static const int forced = env_choice("NVA_ATTN_STREAM");
+  if (forced == 0 || max_q > qtile || num_seqs > kMaxSeqGroups * kWave) return false;
+  return fp8 ? max_q * group <= 32 : forced == 1 && max_q * group <= 16;
+}
+
 bool stream_mode(int32_t num_seqs, int32_t hkv, int32_t max_q, int32_t max_k, int32_t qtile,
                  int32_t group, bool fp8) {
   static const int forced = env_choice("NVA_ATTN_STREAM");
-  if (forced == 0 || max_q > qtile || num_seqs > kMaxSeqGroups * kWave) return false;
-  if (forced == 1) return max_q * group <= (fp8 ? 32 : 16);
-  if (!fp8 || max_q * group > 32) return false;
-  return static_cast<int64_t>(num_seqs) * hkv * max_k >
-         (max_k <= 4096 ? 600 : 480) * static_cast<int64_t>(4 * device_cus());
+  if (!stream_takes(num_seqs, max_q, qtile, group, fp8)) return false;
+  return forced == 1 || static_cast<int64_t>(num_seqs) * hkv * max_k >
+                            (max_k <= 4096 ? 600 : 480) * static_cast<int64_t>(4 * device_cus());
 }
 
 bool pipelined(int nt, bool fp8) {
@@ -2001,14 +2006,18 @@ size_t partials_bytes(int32_t num_tokens, int32_t hq, int32_t max_splits) {
 }
 
 // Workspace for either KV dtype (the size query does not name one): the
-// larger of the stream and fixed layouts that could apply to either.
+// larger of the stream and fixed layouts that could apply to either.  The
+// stream layout counts wherever it is taken at all, also below the batches
+// that prefer it: its bound of a split per 128 keys then covers every smaller
+// batch of the same rows and contexts, which a caller who sizes a workspace
+// for its largest batch goes by.
 size_t workspace_bytes(int32_t num_seqs, int32_t num_tokens, int32_t hq, int32_t hkv, int32_t max_q,
                        int32_t max_k) {
   const int32_t qtile = choose_qtile(max_q, hkv > 0 ? hq / hkv : 1);
   const int32_t group = hkv > 0 ? hq / hkv : 1;
   size_t bytes = 0;
-  if (stream_mode(num_seqs, hkv, max_q, max_k, qtile, group, false) ||
-      stream_mode(num_seqs, hkv, max_q, max_k, qtile, group, true)) {
+  if (stream_takes(num_seqs, max_q, qtile, group, false) ||
+      stream_takes(num_seqs, max_q, qtile, group, true)) {
     bytes = partials_bytes(num_tokens, hq, stream_max_splits(max_k));
   }
   const int32_t n_qtiles = (max_q + qtile - 1) / qtile;
