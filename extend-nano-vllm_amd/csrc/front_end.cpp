@@ -95,9 +95,14 @@ at::Tensor empty_bf16(at::IntArrayRef sizes, const at::Tensor& like) {
   return at::empty(sizes, at::TensorOptions().dtype(at::kBFloat16).device(like.device()));
 }
 
-// The current stream of the current device, as the Python path takes it.
-void* current_stream() {
+// The current stream of the current device, as the Python path takes it;
+// `only` >= 0 leaves another current device to the general path.
+void* current_stream(int64_t only = -1) {
   PyObject* dev = PyObject_CallNoArgs(g_current_device);
+  if (dev && only >= 0 && PyLong_AsLongLong(dev) != only) {
+    Py_DECREF(dev);
+    throw Other{};
+  }
   PyObject* s = dev ? PyObject_CallOneArg(g_raw_stream, dev) : nullptr;
   Py_XDECREF(dev);
   void* p = s ? PyLong_AsVoidPtr(s) : nullptr;
@@ -454,8 +459,8 @@ PyObject* linear(PyObject*, PyObject* const* v, Py_ssize_t n) {
       if (nva_linear_preferred(rows, m, k) && x.stride(0) % 8 == 0 && x.stride(0) >= k &&
           reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
           reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0) {
+        void* s = current_stream(a.device);   // the library's product follows x's device
         at::Tensor out = empty_bf16({rows, m}, x);
-        void* s = current_stream();
         launch([&] {
           return nva_linear(x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), m, rows, m, k, s);
         });
