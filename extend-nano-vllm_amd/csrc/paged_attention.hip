@@ -1186,8 +1186,8 @@ paged_attention_tile_kernel(AttnParams p) {
 //   * K/V tiles are loaded into registers two steps ahead, staged (FP8:
 //     dequantised to bf16) into one of two LDS buffers one step ahead, with
 //     one barrier per step.  Rows of 68 dwords for K (16-byte reads of 8 rows
-//     cover all banks) and 72 for V (a 16-lane transpose load reads four rows
-//     of 32 bytes, 8 banks apart).
+//     cover all banks) and 80 for V (16 lanes of a transpose load read four
+//     rows of 32 bytes, 16 banks apart; the next 16 lanes fill the gaps).
 //   * The heaviest query tiles (the last ones, under the causal mask) are
 //     dispatched first, and the kv head is the fastest grid dimension, so
 //     that with eight kv heads an XCD's L2 holds one head's pages.
@@ -2180,8 +2180,8 @@ int run_attention(AttnParams& p, int kv_dtype, void* workspace, size_t workspace
     p.pair_rows = device_cus() / p.hkv;
     grid = dim3(p.hkv, p.num_seqs, 1);
   } else {
-    choose_split(p.num_seqs, p.hkv, p.max_k, wps, !fp8 && nt >= 4 && tile_choice().wpt, p.block_size, &p.split_len,
-                 &p.max_splits);
+    choose_split(p.num_seqs, p.hkv, p.max_k, wps, !fp8 && nt >= 4 && tile_choice().wpt,
+                 p.block_size, &p.split_len, &p.max_splits);
     // the kernel keeps one block id per lane: a split may touch at most kWave blocks
     if (p.split_len / p.block_size + 2 > kWave) return NVA_ERR_UNSUPPORTED;
     grid = dim3(p.hkv, p.num_seqs, p.max_splits);
