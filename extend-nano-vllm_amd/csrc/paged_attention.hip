@@ -1545,7 +1545,8 @@ paged_attention_wide_kernel(AttnParams p) {
       if (h == 0) p.ws_lse[slot] = lsum > 0.0f ? m_run + __log2f(lsum) : -INFINITY;
     }
   }
-  if (clip_owner) clear_clipped_rows(p, q_start, q_len, q_raw, threadIdx.x, blockDim.x);
+  // by the threads that get here: the other key group has returned
+  if (clip_owner) clear_clipped_rows(p, q_start, q_len, q_raw, tid, kThreads);
 }
 
 // Balanced ("stream") decomposition for one query tile per sequence (verify

@@ -1210,6 +1210,69 @@ def test_several_query_tiles_skip_invalid_blocks_and_scale(K, cuda, fp8):
     assert err <= ATTN_TOL, err
 
 
+def _one_head_each(hq, hkv):
+    """A query head of every kv head, at another place in each group (the
+    oracle's cost is one head in a group's)."""
+    g = hq // hkv
+    return [h * g + (3 * h + 1) % g for h in range(hkv)]
+
+
+# (name, clip_to, paged_case arguments): the wide-tile kernel's instances as
+# 256 CUs pick them (128-row tiles times kv heads against the CUs), query rows
+# past clip_to in some sequences, none in others, one sequence without rows
+WIDE_CLIPPED = [
+    # 23 and 25 tiles, 8 kv heads: two key groups, whole sequences
+    ("two_groups_32_heads", 140, dict(q_len=[150, 141, 139, 0, 160], ctx_lo=150, ctx_hi=400, hq=32,
+                                      hkv=8)),
+    ("two_groups_64_heads", 70, dict(q_len=[80, 71, 69, 100, 75], ctx_lo=70, ctx_hi=300, hq=64, hkv=8)),
+    # one or two tiles: two key groups and key splits
+    ("splits_16_heads", 40, dict(q_len=[45, 40], ctx_lo=600, ctx_hi=900, hq=16, hkv=8)),
+    ("splits_32_heads", 30, dict(q_len=[33, 12, 31], ctx_lo=700, ctx_hi=900, hq=32, hkv=8)),
+    ("splits_64_heads", 15, dict(q_len=[16, 0, 20], ctx_lo=1900, ctx_hi=2100, hq=64, hkv=8)),
+    # 36 tiles under 1024 keys: four waves, one key group
+    ("four_waves_32_heads", 70, dict(q_len=[80, 71, 70, 69, 1, 90] * 2, ctx_lo=70, ctx_hi=300, hq=32,
+                                     hkv=8, block_size=32)),
+    ("four_waves_64_heads", 33, dict(q_len=[40, 34, 33, 32, 1, 45] * 2, ctx_lo=33, ctx_hi=200, hq=64,
+                                     hkv=8, block_size=32)),
+    # 65 tiles of one sequence: eight waves
+    ("eight_waves", 257, dict(q_len=[300], ctx_lo=310, ctx_hi=310, hq=128, hkv=4)),
+]
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("name,clip_to,kw", WIDE_CLIPPED, ids=[c[0] for c in WIDE_CLIPPED])
+def test_rows_past_max_seqlen_q_are_cleared_with_several_query_tiles(K, cuda, name, clip_to, kw, fp8):
+    """As test_rows_past_max_seqlen_q_are_cleared, where max_seqlen_q spans
+    several 64-row query tiles: every head of a row past it is zero, whatever
+    out and the workspace held before, and the kept rows are the oracle's with
+    their unclipped windows."""
+    case = paged_case(seed=22, batch=len(kw["q_len"]), **kw)
+    kc, vc = case["k_cache"], case["v_cache"]
+    if fp8:
+        kc, vc = kc.float().to(torch.float8_e4m3fn), vc.float().to(torch.float8_e4m3fn)
+    args = (kc.to(cuda), vc.to(cuda), case["cu_q"].to(cuda), case["cu_k"].to(cuda))
+    q, bt, max_k = case["q"].to(cuda), case["block_tables"].to(cuda), int(case["lens"].max())
+    K.paged_attention_varlen(q, *args, max(case["q_lens"]), max_k, 128 ** -0.5, bt)   # stale counts
+    out = torch.full_like(q, 7.0)
+    K.paged_attention_varlen(q, *args, clip_to, max_k, 128 ** -0.5, bt, out=out)
+    torch.cuda.synchronize()
+    got, cu = out.float().cpu(), case["cu_q"].tolist()
+    rows, kept, lens = [], [], []
+    for i, (qn, L) in enumerate(zip(case["q_lens"], case["lens"].tolist())):
+        keep = min(qn, clip_to)
+        rows += range(cu[i], cu[i] + keep)
+        kept.append(keep)
+        lens.append(L - (qn - keep))
+        heads = got[cu[i] + keep:cu[i + 1]].abs().amax((0, 2)) if qn > keep else torch.zeros(1)
+        assert heads.nonzero().flatten().tolist() == [], (name, i, "heads not cleared")
+    rows, pick = torch.tensor(rows), _one_head_each(kw["hq"], kw["hkv"])
+    ref = oracle.paged_attention(bits(case["q"][rows][:, pick]), bits(kc), bits(vc),
+                                 np.array([0] + np.cumsum(kept).tolist(), np.int32),
+                                 np.array(lens, np.int32), case["block_tables"].numpy(), 128 ** -0.5)
+    err = np.abs(got[rows][:, pick].numpy() - ref).max()
+    assert err <= ATTN_TOL, (name, err)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("hq,q_len", [(8, [1, 1, 0, 1, 1]), (32, [6, 3, 1, 6, 2]), (64, [8, 8, 5, 8, 0])])
 def test_small_batch_decompositions(K, cuda, hq, q_len, fp8):
