@@ -114,14 +114,20 @@ void* current_stream(int64_t only = -1) {
   return p;
 }
 
-// Runs a C-ABI call without the interpreter lock; a refused call is the
-// general path's to report.
+struct WithoutGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
+// Runs a C-ABI call without the interpreter lock (taken again also where `f`
+// throws); a refused call is the general path's to report.
 template <typename F>
 void launch(F&& f) {
   int status;
-  Py_BEGIN_ALLOW_THREADS
-  status = f();
-  Py_END_ALLOW_THREADS
+  {
+    WithoutGil free;
+    status = f();
+  }
   need(status == NVA_OK);
 }
 
@@ -200,7 +206,7 @@ PyObject* rms_norm(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const at::Tensor& x = a.tensor(0);
     const at::Tensor& w = a.tensor(1);
     need_rows(x);
-    const int64_t rows = x.size(0), h = x.size(1);
+    const int32_t rows = as_i32(x.size(0)), h = as_i32(x.size(1));
     need(w.numel() == h);
     at::Tensor out;
     if (a.none(3)) {
@@ -213,8 +219,8 @@ PyObject* rms_norm(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const float eps = a.f32(2);
     void* s = current_stream();
     launch([&] {
-      return nva_rms_norm(x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), out.stride(0),
-                          as_i32(rows), as_i32(h), eps, s);
+      return nva_rms_norm(x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), out.stride(0), rows,
+                          h, eps, s);
     });
     return THPVariable_Wrap(out);
   });
@@ -285,6 +291,7 @@ PyObject* qk_norm_rope_store(PyObject*, PyObject* const* v, Py_ssize_t n) {
     const int32_t t = as_i32(qkv.size(0));
     need(pos.scalar_type() == at::kLong && pos.is_contiguous() && pos.numel() == t);
     need(cs.scalar_type() == at::kFloat && cs.is_contiguous() && cs.dim() >= 1);
+    const int32_t max_pos = as_i32(cs.size(0));
     need(p.hkv == hkv && p.d == d && hq >= 0 && hkv >= 0 && d >= 0);
     need(qkv.size(1) >= (static_cast<int64_t>(hq) + 2 * static_cast<int64_t>(hkv)) * d);
     need_i32(slots);
@@ -294,7 +301,7 @@ PyObject* qk_norm_rope_store(PyObject*, PyObject* const* v, Py_ssize_t n) {
     launch([&] {
       return nva_qk_norm_rope_store(
           qkv.data_ptr(), qkv.stride(0), static_cast<const int64_t*>(pos.data_ptr()), qw, kw,
-          static_cast<const float*>(cs.data_ptr()), as_i32(cs.size(0)), t, hq, hkv, d, eps,
+          static_cast<const float*>(cs.data_ptr()), max_pos, t, hq, hkv, d, eps,
           q.data_ptr(), p.k, p.v, p.kv_dtype, p.blk, p.tok, p.head, p.num_blocks, p.block_size,
           static_cast<const int32_t*>(slots.data_ptr()), ks, vs, s);
     });
@@ -305,7 +312,7 @@ PyObject* qk_norm_rope_store(PyObject*, PyObject* const* v, Py_ssize_t n) {
 // What the two attention entry points share.
 struct Attention {
   Pages p;
-  int32_t t, hq;
+  int32_t t, hq, bt_cols;
   at::Tensor out;
 };
 Attention attention(Args& a, const at::Tensor& q, int ki, int vi, const at::Tensor& bt, int out_i) {
@@ -316,6 +323,7 @@ Attention attention(Args& a, const at::Tensor& q, int ki, int vi, const at::Tens
   need(bt.scalar_type() == at::kInt && bt.dim() == 2 && bt.stride(1) == 1);
   r.t = as_i32(q.size(0));
   r.hq = as_i32(q.size(1));
+  r.bt_cols = as_i32(bt.size(1));
   if (a.none(out_i)) {
     r.out = empty_bf16(q.sizes(), q);
   } else {
@@ -352,7 +360,7 @@ PyObject* paged_attention_varlen(PyObject*, PyObject* const* v, Py_ssize_t n) {
           q.data_ptr(), q.stride(0), q.stride(1), r.p.k, r.p.v, r.p.kv_dtype, r.p.blk, r.p.tok,
           r.p.head, r.p.num_blocks, r.p.block_size, static_cast<const int32_t*>(cu_q.data_ptr()),
           static_cast<const int32_t*>(cu_k.data_ptr()), static_cast<const int32_t*>(bt.data_ptr()),
-          bt.stride(0), as_i32(bt.size(1)), b, r.t, max_q, max_k, r.hq, r.p.hkv, r.p.d, scale, ks, vs,
+          bt.stride(0), r.bt_cols, b, r.t, max_q, max_k, r.hq, r.p.hkv, r.p.d, scale, ks, vs,
           r.out.data_ptr(), r.out.stride(0), r.out.stride(1), w.ptr, w.bytes, s);
     });
     return THPVariable_Wrap(r.out);
@@ -373,7 +381,7 @@ PyObject* paged_attention_decode(PyObject*, PyObject* const* v, Py_ssize_t n) {
     need_i32(lens);
     const Attention r = attention(a, q, 1, 2, bt, 9);
     need(lens.numel() == r.t && bt.size(0) >= r.t);
-    const int32_t max_k = a.none(6) ? as_i32(bt.size(1) * r.p.block_size) : a.i32(6);
+    const int32_t max_k = a.none(6) ? as_i32(int64_t{r.bt_cols} * r.p.block_size) : a.i32(6);
     const Workspace w = workspace(
         v[10], a.device,
         nva_paged_attention_workspace_size(r.t, r.t, r.hq, r.p.hkv, r.p.d, 1, max_k));
@@ -382,7 +390,7 @@ PyObject* paged_attention_decode(PyObject*, PyObject* const* v, Py_ssize_t n) {
       return nva_paged_attention_decode(
           q.data_ptr(), q.stride(0), q.stride(1), r.p.k, r.p.v, r.p.kv_dtype, r.p.blk, r.p.tok,
           r.p.head, r.p.num_blocks, r.p.block_size, static_cast<const int32_t*>(lens.data_ptr()),
-          static_cast<const int32_t*>(bt.data_ptr()), bt.stride(0), as_i32(bt.size(1)), r.t, max_k,
+          static_cast<const int32_t*>(bt.data_ptr()), bt.stride(0), r.bt_cols, r.t, max_k,
           r.hq, r.p.hkv, r.p.d, scale, ks, vs, r.out.data_ptr(), r.out.stride(0), r.out.stride(1),
           w.ptr, w.bytes, s);
     });
@@ -437,11 +445,6 @@ bool watched() {
   return c10::impl::TorchDispatchModeTLS::any_modes_set() || torch::jit::tracer::isTracing() ||
          at::autocast::is_autocast_enabled(at::kCUDA);
 }
-
-struct WithoutGil {
-  PyThreadState* state = PyEval_SaveThread();
-  ~WithoutGil() { PyEval_RestoreThread(state); }
-};
 
 // (x, weight, bias | None) -> x weight^T + bias: few rows without a bias on the
 // kernel of linear.hip, everything else the library's product

@@ -151,6 +151,24 @@ def test_attention_equals_the_python_path(cuda, monkeypatch, fp8, head_major):
         _same(*_both(monkeypatch, decode))
 
 
+@pytest.mark.gpu
+def test_sizes_past_32_bits_are_handed_off(cuda):
+    """More rows than a C-ABI count holds (views of one row, no memory behind
+    them): the front end hands the call back with the interpreter as it was,
+    and the Python path refuses it."""
+    f = _native.load_front_end()
+    row = torch.ones(1, 8, device=cuda).to(BF16)
+    w, out = torch.ones(8, device=cuda).to(BF16), torch.zeros(1, 8, device=cuda).to(BF16)
+    n = 2 ** 31
+    assert f.rms_norm(row.expand(n, 8), w, 1e-6, out.expand(n, 8)) is None
+    with pytest.raises(ValueError):
+        K.rms_norm(row.expand(n, 8), w, 1e-6, out=out.expand(n, 8))
+    assert f.silu_mul(row.expand(n, 8)) is None
+    assert f.add_rms_norm(row.expand(n, 8), row.expand(n, 8), w, 1e-6) is None
+    assert f.argmax_rows(row.expand(n, 8), None, None, {}) is None
+    assert K.rms_norm(row, w, 1e-6).shape == (1, 8)
+
+
 LINEAR_SHAPES = [
     # rows around the 16-row tiles and the limit, K of one chunk, fewer chunks
     # than waves, a remainder of waves and of depth, N short of a tile
