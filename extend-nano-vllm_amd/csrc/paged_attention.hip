@@ -1769,29 +1769,47 @@ TileChoice tile_choice() {
 // 56.6 at 2432.
 // Fewer segments than the device has places for (a place: a CU for eight-wave
 // segments, half a CU for shared tiles, a SIMD for single waves) take splits
-// of an even share of the longest sequence: about as many segments as places,
-// in one round.  Eight-wave and shared-tile splits round the share count to
-// the nearer (eight waves: two thirds up), since the lengths spread below the
-// longest and a second round costs more than idle CUs (Qwen3-0.6B decode, 24
-// sequences of 300-1000 keys: 17.4 us whole, 22.8 in halves).  Below 256 keys
-// a split gives waves nothing to do, and 32 splits of 128 cost the combine
-// more than they save (4000 keys 13.4 against 12.1), so long sequences stop
-// there, the shortest stay whole (300 keys 8.0 against 8.9 in three), and
-// 64-row tiles over more than 8192 keys stop at 512 (16000: 27.1 against
-// 33.5).  Until about 1024 waves ran at all, lengths used to shrink from the
-// default; measured against that, us per call, one box, alternating:
-//   Qwen3-0.6B decode: 4 x 1000-2000 keys 15.0 -> 13.0, 4 x 4000-8000 33.9 ->
-//   23.2, 8 x 500-1500 20.5 -> 13.5, 12 x 1000-3000 33.4 -> 26.0;
-//   Qwen3-8B verify (6 rows): 4 x 4000-8000 36.8 -> 27.9, 12 x 1000-3000 37.0
-//   -> 25.7; Qwen3-32B verify (8 rows): 1 x 16000 42.8 -> 27.1, 24 x 300-1000
-//   36.4 -> 30.4, 48 x 300-1200 47.7 -> 39.6, FP8 64 x 500-3000 194 -> 115;
-//   slower only 8 x 2000-8000 at 64 rows, 46.0 -> 47.8.
+// of an even share of the longest sequence, as many as fill one round.  A
+// share too many costs a second round when the lengths are equal, a share too
+// few leaves places empty when they spread below the longest; the host knows
+// neither, so the lines below lie where the equal lengths (first figure: r 1)
+// lose nothing and the spread ones (r 4: lengths from a quarter of the
+// longest) keep what they can.  us, whole places only / one share more:
+//   * eight waves: 144 segments of 1000 keys 18.1 whole / 28.1 halves, 24 of
+//     2600 12.6 in ten / 15.7 in eleven.  Two shares become three where they
+//     overflow the round by at most an eighth: 96 segments of 2600 r 4 22.7 /
+//     18.9, r 1 27.3 / 31.6 (whole 35); past 2816 keys, the default split, no
+//     more (4400 keys r 1 40 / 48).  Up to 512 keys, and up to 896 in three
+//     shares or fewer, sequences stay whole (96 of 600: 12.8 / 18.7; 128 of
+//     600: 12.2 / 14.7); a share has at least 256 keys past 1024 (4000 keys:
+//     32 splits of 128 cost the combine 13.4 against 12.1 in all).
+//   * shared tiles: the nearer count, but one less where it overflows the
+//     round by more than a sixteenth (184 segments of 2600-8000 keys r 1 57.0,
+//     137 / 62.4, 161; r 4 level), for two shares only up to 2304 keys (288 of
+//     2100: 70.4 / 74.4; of 2600 r 4 65 / 53).  Shares have at least 256 keys
+//     past 2048 (one sequence past 3328) and 512 past 8192 (16000: 27.1
+//     against 33.5 in 128s).
+//   * single waves of more than 32 rows (FP8 verify tiles of 64): a wave's time
+//     is its keys', so a second round costs a whole share (160 segments of
+//     16000 keys r 1 191 / 302, 240 of 8000 150 / 214).  Places that stay idle
+//     take a shorter last share instead, a k-th of the others where k of them
+//     one after the other serve every segment, k up to 4 (400 segments of 4400
+//     keys r 1: 163 in two shares, 191 in three, 138 in two and a half).  Up to
+//     1024 keys, where a share is short, one more pays when lengths spread
+//     (400 of 600 r 2 42.7 / 37.1), also halves of 1024-3328 keys (640 of 3200
+//     r 4 151 / 124, r 1 160 / 218, whole 212); nine shares or more hide it.
+//   * single waves of up to 32 rows share a SIMD two by two: one share more.
+// Against the rule of at least 1024 waves that shrank the default length
+// before, alternating on one box, us: Qwen3-0.6B decode 4 x 4000-8000 keys 33.9
+// -> 23.2, 8 x 500-1500 20.5 -> 13.5; Qwen3-8B verify (6 rows) 4 x 4000-8000
+// 36.8 -> 27.9; Qwen3-32B verify (8 rows) 1 x 16000 42.8 -> 27.1, 48 x 300-1200
+// 47.7 -> 39.6, FP8 64 x 500-3000 194 -> 115.
 // The length is capped so that a split spans at most kWave - 2 blocks of
 // block_size tokens (the kernel holds one block id per lane); block_size 0
 // (unknown: the workspace query) assumes the smallest block, kChunk tokens,
 // which bounds the split count from above.
-void choose_split(int32_t num_seqs, int32_t num_kv_heads, int32_t max_k, int32_t waves, bool tile,
-                  int32_t block_size, int32_t* split_len, int32_t* max_splits) {
+void choose_split(int32_t num_seqs, int32_t num_kv_heads, int32_t max_k, int32_t waves, int nt,
+                  bool tile, int32_t block_size, int32_t* split_len, int32_t* max_splits) {
   const int64_t segs = static_cast<int64_t>(num_seqs > 0 ? num_seqs : 1) *
                        (num_kv_heads > 0 ? num_kv_heads : 1);
   const int32_t mk = max_k > 1 ? max_k : 1;
@@ -1808,16 +1826,34 @@ void choose_split(int32_t num_seqs, int32_t num_kv_heads, int32_t max_k, int32_t
   }
   const int32_t span = (kWave - 2) * (block_size > 0 ? block_size : kChunk);
   if (len > span) len = span / kMinSplit * kMinSplit;
-  const int64_t want = (waves > 1 ? 1 : tile ? 2 : 4) * static_cast<int64_t>(cus);
-  const int64_t parts = waves > 1 ? (3 * want + segs) / (3 * segs)
-                        : tile    ? (2 * want + segs) / (2 * segs)
-                                  : (want + segs - 1) / segs;
-  if (parts > 1) {
-    const int32_t up = waves > 1 || tile ? kMinSplit - 1 : kMinSplit / 2;
-    int32_t even = static_cast<int32_t>(((mk + parts - 1) / parts + up) / kMinSplit * kMinSplit);
-    const int32_t least = waves > 1 ? (mk <= 384 ? whole : mk <= 1024 ? kMinSplit : 2 * kMinSplit)
-                          : tile    ? (mk <= 2048 ? kMinSplit : mk <= 8192 ? 2 * kMinSplit : 4 * kMinSplit)
-                                    : (mk <= 8192 ? kMinSplit : 2 * kMinSplit);
+  const int64_t places = (waves > 1 ? 1 : tile ? 2 : 4) * static_cast<int64_t>(cus);
+  int64_t parts = places / segs, last = 0;      // shares that fill one round
+  int32_t round_up = kMinSplit - 1, least;
+  if (waves > 1) {
+    if (parts == 2 && 8 * 3 * segs <= 9 * places && mk <= 2816) parts = 3;
+    least = mk <= 512 || (mk <= 896 && parts <= 3) ? whole : mk <= 1024 ? kMinSplit : 2 * kMinSplit;
+  } else if (tile) {
+    parts = (2 * places + segs) / (2 * segs);
+    if (16 * segs * parts > 17 * places && (parts > 2 || (parts == 2 && mk <= 2304))) --parts;
+    least = mk <= (segs <= 8 ? 3328 : 2048) ? kMinSplit : mk <= 8192 ? 2 * kMinSplit : 4 * kMinSplit;
+  } else {
+    least = mk <= 8192 ? kMinSplit : 2 * kMinSplit;
+    if (nt < 4 || parts >= 9) {
+      parts = (places + segs - 1) / segs;
+      round_up = kMinSplit / 2;
+    } else if (parts > 0 && (mk <= 1024 ? parts > 1 : parts == 1 && mk <= 3328)) {
+      parts = (places + segs - 1) / segs;
+    } else if (parts > 0) {
+      const int64_t idle = places - parts * segs;
+      const int64_t k = idle > 0 ? (segs + idle - 1) / idle : 0;
+      if (k > 0 && k <= 4) last = k;
+    }
+    if (mk <= 384 && (parts < 2 || (parts == 2 && last == 0))) least = whole;
+  }
+  // `parts` shares and, with `last`, one of a last-th of a share
+  if (parts > 1 || last > 0) {
+    const int64_t num = mk * (last > 0 ? last : 1), den = last > 0 ? parts * last + 1 : parts;
+    int32_t even = static_cast<int32_t>(((num + den - 1) / den + round_up) / kMinSplit * kMinSplit);
     if (even < least) even = least;
     if (even < len) len = even;
   }
@@ -2030,8 +2066,9 @@ size_t workspace_bytes(int32_t num_seqs, int32_t num_tokens, int32_t hq, int32_t
   const int nt = tile_mfmas(qtile * (hkv > 0 ? hq / hkv : 1));
   // either KV dtype: the larger split count of the two wave choices
   int32_t len, ms, ms_fp8;
-  choose_split(num_seqs, hkv, max_k, segment_waves(nt, false), tile_choice().wpt && nt >= 4, 0, &len, &ms);
-  choose_split(num_seqs, hkv, max_k, segment_waves(nt, true), false, 0, &len, &ms_fp8);
+  choose_split(num_seqs, hkv, max_k, segment_waves(nt, false), nt, tile_choice().wpt && nt >= 4, 0,
+               &len, &ms);
+  choose_split(num_seqs, hkv, max_k, segment_waves(nt, true), nt, false, 0, &len, &ms_fp8);
   ms = ms_fp8 > ms ? ms_fp8 : ms;
   if (ms > 1) {
     const size_t fixed = partials_bytes(num_tokens, hq, ms);
@@ -2181,7 +2218,7 @@ int run_attention(AttnParams& p, int kv_dtype, void* workspace, size_t workspace
     p.pair_rows = device_cus() / p.hkv;
     grid = dim3(p.hkv, p.num_seqs, 1);
   } else {
-    choose_split(p.num_seqs, p.hkv, p.max_k, wps, !fp8 && nt >= 4 && tile_choice().wpt,
+    choose_split(p.num_seqs, p.hkv, p.max_k, wps, nt, !fp8 && nt >= 4 && tile_choice().wpt,
                  p.block_size, &p.split_len, &p.max_splits);
     // the kernel keeps one block id per lane: a split may touch at most kWave blocks
     if (p.split_len / p.block_size + 2 > kWave) return NVA_ERR_UNSUPPORTED;
