@@ -2005,9 +2005,21 @@ int32_t stream_ranges_per_head(int32_t hkv) {
 //     prompts at Qwen3-8B 1129 -> 1091, 4096-token ones 606 -> 582,
 //     Qwen3-0.6B FP8 316 -> 300; short ones stay at four (256-2048 tokens,
 //     FP8 0.6B, 129 against 151).
-//   * key splits while there are fewer groups than CUs (a verify of more than
-//     64 rows over long contexts): 72 rows over 16000 keys 29 us split against
-//     ~240 whole (8 groups), 55 with the 64-row tiles.
+//   * up to 128 keys, one or two steps, one key group: a second one only adds
+//     the fold (60 keys 8.5 -> 6.9, 100 keys 9.2 -> 8.7).  Up to 256 keys, and
+//     to 384 or 640 where there are more than 32 or 64 groups, whole sequences:
+//     the combine costs what the splits save (200 keys, 64 groups 18.3 -> 12.3).
+//   * longer ones are split while there are fewer groups than CUs (a verify of
+//     more than 64 rows): splits of 1024 keys or more as many as two workgroups
+//     a CU take, with one key group (a workgroup beside another hides what the
+//     second group would; lengths from a quarter of the longest: 96 groups of
+//     5000 keys 62.8 -> 49.4, 136 of 16000 310 -> 176, where the 64-row tiles
+//     took 62 and 258), shorter ones as many as one a CU, with two key groups
+//     (64 groups of 2400 keys: 28.0, in 640-key splits of one group 29.6; a
+//     bound far above the lengths leaves few splits, 4 x 600-800 keys under
+//     4832: 22.6, one group 30.8).  Halves only of up to 192 groups past 6144
+//     keys (240 of 3200 equal ones: 63 whole, 75).  Splits of 128 keys take one
+//     group.  72 rows over 16000 keys: 27 us (~240 whole, 53 on the 64-row tiles).
 struct WidePlan {
   int32_t waves, key_groups, qtile, n_qtiles, split_len, max_splits;
 };
@@ -2023,14 +2035,27 @@ WidePlan wide_plan(int32_t num_seqs, int32_t num_tokens, int32_t hkv, int32_t gr
   const int64_t groups = tiles * hkv;
   w.waves = 4;
   w.key_groups = 1;
-  if (groups <= cus || (groups <= 2 * cus && mk >= 1024))
-    w.key_groups = 2;
-  else if (rows >= 8192 * static_cast<int64_t>(num_seqs))
-    w.waves = 8;
+  int64_t len = mk;
+  if (groups > cus) {
+    if (groups <= 2 * cus && mk >= 1024)
+      w.key_groups = 2;
+    else if (rows >= 8192 * static_cast<int64_t>(num_seqs))
+      w.waves = 8;
+  } else if (mk > 128) {
+    const int64_t parts = cus / groups, pairs = 2 * cus / groups;
+    const int64_t half = (mk + pairs - 1) / pairs;
+    if (mk <= 256 || (mk <= 384 && groups > 32) || (mk <= 640 && groups >= 64)) {
+      w.key_groups = 2;
+    } else if (half > 1024 - kMinSplit &&
+               (pairs > 2 ? mk > 2048 : mk > 6144 && 4 * groups <= 3 * cus)) {
+      len = half;
+    } else {
+      len = (mk + parts - 1) / parts;
+      w.key_groups = len > kMinSplit ? 2 : 1;
+    }
+  }
   w.qtile = 32 * w.waves / group;
   w.n_qtiles = (max_q + w.qtile - 1) / w.qtile;
-  const int64_t parts = groups < cus ? cus / groups : 1;
-  const int64_t len = (mk + parts - 1) / parts;
   w.split_len = static_cast<int32_t>((len + kMinSplit - 1) / kMinSplit * kMinSplit);
   w.max_splits = (mk + w.split_len - 1) / w.split_len;
   return w;

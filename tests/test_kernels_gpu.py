@@ -1168,6 +1168,79 @@ WIDE_CASES = [
 ]
 
 
+# One query head of every kv head against the oracle: more rows and keys than
+# WIDE_CASES, at every instance (four waves with one and two key groups, eight
+# waves) with and without key splits, as 256 CUs pick them
+WIDE_LARGE = [
+    # packed prompts, 51 tiles of 128 rows under 1024 keys: four waves, one group
+    ("four_waves", dict(q_len=[37, 129, 5, 64, 33, 100, 1, 0, 90, 16, 17, 48, 77], ctx_lo=1, ctx_hi=200,
+                        hq=64, hkv=8, block_size=32)),
+    # 65 sequences, one of them past the 64 page ids a wave holds at once
+    ("four_waves_pages", dict(q_len=[16] * 65, ctx_lo=16, ctx_hi=60, hq=64, hkv=8, block_size=32,
+                              first=2500)),
+    # one sequence of 65 tiles past the 64 page ids
+    ("eight_waves_pages", dict(q_len=[257], ctx_lo=2100, ctx_hi=2100, hq=256, hkv=8, block_size=32)),
+    # short sequences: one step, two steps, the first past them
+    ("64_keys", dict(q_len=[30, 17, 64, 0, 1], ctx_lo=64, ctx_hi=64, hq=64, hkv=8, block_size=32)),
+    ("128_keys", dict(q_len=[30, 17, 90, 128], ctx_lo=128, ctx_hi=128, hq=64, hkv=8, block_size=32)),
+    ("129_keys", dict(q_len=[30, 17, 90, 128], ctx_lo=129, ctx_hi=129, hq=64, hkv=8, block_size=32)),
+    # splits of 128 keys, four waves and one group
+    ("splits_one_group", dict(q_len=[12, 9], ctx_lo=1000, ctx_hi=1100, hq=64, hkv=8, block_size=64)),
+    # splits of two workgroups a CU: 80 and 176 groups
+    ("long_splits", dict(q_len=[20, 9, 17, 24, 3], ctx_lo=1500, ctx_hi=4000, hq=64, hkv=8)),
+    ("long_halves", dict(q_len=[17] * 10 + [200], ctx_lo=200, ctx_hi=900, hq=32, hkv=8, block_size=32,
+                         first=6500)),
+]
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("name,kw", WIDE_LARGE, ids=[c[0] for c in WIDE_LARGE])
+def test_several_query_tiles_at_every_instance(K, cuda, name, kw, fp8):
+    """Sequences of several 64-row query tiles against the oracle, a page of
+    an invalid id (its keys unseen by every tile) among the longest one's."""
+    kw = dict(kw)
+    first = kw.pop("first", None)
+    case = paged_case(seed=23, batch=len(kw["q_len"]), **kw)
+    lens, bt = case["lens"].clone(), case["block_tables"]
+    kc, vc = case["k_cache"], case["v_cache"]
+    bs = case["block_size"]
+    if first:                        # the first sequence's pages: all the others', over and over
+        n = -(-first // bs)
+        longer = torch.full((bt.shape[0], n + 1), -1, dtype=torch.int32)
+        longer[:, :bt.shape[1]] = bt
+        longer[0, :n] = torch.arange(n, dtype=torch.int32) * 7 % kc.shape[0]
+        bt, lens[0] = longer, first
+    if fp8:
+        kc, vc = kc.float().to(torch.float8_e4m3fn), vc.float().to(torch.float8_e4m3fn)
+    cu_k = torch.tensor([0] + np.cumsum(lens.tolist()).tolist(), dtype=torch.int32)
+    args = (case["q"].to(cuda), kc.to(cuda), vc.to(cuda), case["cu_q"].to(cuda), cu_k.to(cuda),
+            max(case["q_lens"]), int(lens.max()), 128 ** -0.5)
+    pick = _one_head_each(kw["hq"], kw["hkv"])
+    q = case["q"][:, pick]
+
+    def check(tables, oracle_lens, oracle_tables):
+        out = K.paged_attention_varlen(*args, tables.to(cuda))
+        again = K.paged_attention_varlen(*args, tables.to(cuda))
+        torch.cuda.synchronize()
+        assert torch.equal(out, again), name
+        ref = oracle.paged_attention(bits(q), bits(kc), bits(vc), case["cu_q"].numpy(),
+                                     oracle_lens.numpy(), oracle_tables.numpy(), 128 ** -0.5)
+        err = np.abs(out[:, pick].float().cpu().numpy() - ref).max()
+        assert err <= ATTN_TOL, (name, err)
+
+    check(bt, lens, bt)
+    # an invalid page before the longest sequence's query rows
+    i = int(lens.argmax())
+    gone = (int(lens[i]) - case["q_lens"][i]) // bs - 1
+    if gone < 0:
+        return
+    bad, cut, short = bt.clone(), bt.clone(), lens.clone()
+    bad[i, gone] = kc.shape[0] + 3
+    cut[i, gone:-1] = bt[i, gone + 1:]
+    short[i] -= bs
+    check(bad, short, cut)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("name,kw", WIDE_CASES, ids=[c[0] for c in WIDE_CASES])
 def test_several_query_tiles(K, cuda, name, kw, fp8):
