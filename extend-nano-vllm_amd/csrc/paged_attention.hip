@@ -6,7 +6,8 @@
 // tile is up to 64/G query positions of a sequence times the G query heads
 // that share the kv head (G = Hq / Hkv), padded to NT*16 columns (NT = 1, 2,
 // 4): every row of a verify step (k+1 positions).  Sequences with more rows
-// than one such tile (prefill) run on the wide-tile kernel below.  Segments
+// than one such tile (prefill) run on the wide-tile kernel below, a few short
+// ones on the shared-tile kernel's 64-row tiles.  Segments
 // come from one of two decompositions:
 //   * stream (single-tile sequences of at most 32 rows over an FP8 cache, in
 //     batches of many keys):
@@ -873,9 +874,11 @@ paged_attention_kernel(AttnParams p) {
 }
 
 // ---------------------------------------------------------------- shared-tile kernel
-// Tiles of 33-64 rows (64-row verify tiles of GQA group 8 with k = 7): WPT
-// waves share one segment (kv head, sequence, key split), wave w owning the NTW = 4 / WPT column
-// tiles 16 NTW w .. of the 64 query columns over every key of the split,
+// Tiles of 33-64 rows (64-row verify tiles of GQA group 8 with k = 7, and the
+// several tiles of a few short sequences, short_tiles): WPT waves share one
+// segment (kv head, sequence, query tile, key split), wave w owning the NTW =
+// 4 / WPT column tiles 16 NTW w .. of the 64 query columns over every key of
+// the split,
 // so each wave finishes its own columns and nothing is merged.
 //   * The workgroup loads each 32-key chunk once, cooperatively: thread t
 //     takes the 16-byte granules t, t + WPT * 64, ... of the chunk's 8 KiB
@@ -906,31 +909,38 @@ paged_attention_tile_kernel(AttnParams p) {
 
   const int kvh = blockIdx.x;
   const int seq = blockIdx.y;
-  const int split = blockIdx.z;
+  int split = blockIdx.z, qt = 0;
+  if (p.n_qtiles > 1) {   // the division costs a single-tile call 0.3 us
+    qt = split / p.max_splits;
+    split -= qt * p.max_splits;
+  }
   const int kv_begin = split * p.split_len;
   const int lane_blk = split_block_ids(p, seq, kv_begin);
   int q_start, q_len, L, q_raw;
   seq_geometry_uniform(p, seq, q_start, q_len, L, &q_raw);
-  const int nsplit = L > 0 ? (L + p.split_len - 1) / p.split_len : 0;
+  const int j0 = qt * p.qtile;
+  const int jn = (q_len - j0 < p.qtile) ? q_len - j0 : p.qtile;
+  const int kv_limit = L - q_len + j0 + jn;  // meaningful when jn > 0
+  const int nsplit = kv_limit > 0 ? (kv_limit + p.split_len - 1) / p.split_len : 0;
   const bool note = kvh == 0 && split == 0 && p.row_nsplit;
-  const bool clip_owner = kvh == 0 && split == 0 && q_raw > q_len;
-  if (q_len <= 0 || kv_begin >= L) {
-    if (q_len > 0) {
-      if (note) note_rows(p, seq, 0, nsplit);
-      if (L <= 0 && split == 0) zero_tile(p, kvh, seq, 0);
+  const bool clip_owner = kvh == 0 && split == 0 && qt == p.n_qtiles - 1 && q_raw > q_len;
+  if (jn <= 0 || kv_begin >= kv_limit) {
+    if (jn > 0) {
+      if (note) note_rows(p, seq, qt, nsplit);
+      if (kv_limit <= 0 && split == 0) zero_tile(p, kvh, seq, qt);
     }
     if (clip_owner) clear_clipped_rows(p, q_start, q_len, q_raw, threadIdx.x, blockDim.x);
     return;
   }
-  if (note) note_rows(p, seq, 0, nsplit);
-  const int kv_end = kv_begin + p.split_len < L ? kv_begin + p.split_len : L;
+  if (note) note_rows(p, seq, qt, nsplit);
+  const int kv_end = kv_begin + p.split_len < kv_limit ? kv_begin + p.split_len : kv_limit;
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int g = lane >> 4;
   const int m16 = lane & 15;
-  const int rows = q_len * p.group;
+  const int rows = jn * p.group;
   const float sl2 = p.scale_log2;
 
   // ---- this wave's query operands (padding columns zero) and causal limits
@@ -940,7 +950,7 @@ paged_attention_tile_kernel(AttnParams p) {
   for (int nt = 0; nt < NTW; ++nt) {
     const int n = (wv * NTW + nt) * 16 + m16;
     const int nn = n < rows ? n : 0;
-    const int j = nn / p.group, hh = nn % p.group;
+    const int j = j0 + nn / p.group, hh = nn % p.group;
     const uint16_t* qp = p.q + static_cast<int64_t>(q_start + j) * p.q_row_stride +
                          static_cast<int64_t>(kvh * p.group + hh) * p.q_head_stride;
 #pragma unroll
@@ -973,7 +983,7 @@ paged_attention_tile_kernel(AttnParams p) {
     const int kb = kv_begin + cc * kChunk;
     const int raw = chunk_block(cc);
     const bool valid = live && raw >= 0 && raw < p.num_blocks;
-    const int visible = L - kb < kChunk ? L - kb : kChunk;
+    const int visible = kv_limit - kb < kChunk ? kv_limit - kb : kChunk;
     const int nrec = valid ? visible * static_cast<int>(tokb) : 0;
     const int64_t tile = (static_cast<int64_t>(valid ? raw : 0) * p.blk_stride +
                           static_cast<int64_t>(kvh) * p.head_stride +
@@ -1031,7 +1041,7 @@ paged_attention_tile_kernel(AttnParams p) {
         for (int kt = 0; kt < 2; ++kt) sacc[kt][nt] = mfma(kop[kt], qv[nt][s], sacc[kt][nt]);
     }
     // masked only past a causal limit, behind a uniform branch (as above)
-    const bool full = kb + kChunk - 1 <= L - q_len && kb + kChunk <= L;
+    const bool full = kb + kChunk - 1 <= L - q_len + j0 && kb + kChunk <= kv_limit;
     if (!full) {
       const int rel = kb + 4 * g;
 #pragma unroll
@@ -1137,7 +1147,7 @@ paged_attention_tile_kernel(AttnParams p) {
     const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
     const int n = (wv * NTW + nt) * 16 + m16;
     if (n < rows) {
-      const int j = n / p.group, hh = n % p.group;
+      const int j = j0 + n / p.group, hh = n % p.group;
       const int tok = q_start + j;
       const int h = kvh * p.group + hh;
       const int64_t slot = (static_cast<int64_t>(tok) * p.hq + h) * p.max_splits + split;
@@ -1167,7 +1177,7 @@ paged_attention_tile_kernel(AttnParams p) {
 }
 
 // ---------------------------------------------------------------- wide-tile kernel
-// Sequences of several query tiles (every prefill): a workgroup of NW waves
+// Sequences of several query tiles (prefill): a workgroup of NW waves
 // takes 32 NW query rows (32 per wave) of one sequence and kv head over a key
 // range, 64 keys a step, on the 32x32x16 MFMA.
 //   * What bounds it: matrix cores and the softmax's vector instructions
@@ -2061,6 +2071,21 @@ WidePlan wide_plan(int32_t num_seqs, int32_t num_tokens, int32_t hkv, int32_t gr
   return w;
 }
 
+// Whether the several 64-row query tiles of a few short sequences (bf16) stay on
+// the shared-tile kernel, in splits of 128 keys: a workgroup of it starts in
+// less time than a wide one (no second key group, a quarter of the keys before
+// its first product), which counts where the whole call is one such step.  Both
+// sides, us (64-row / wide): 8 x 17 rows of 60 keys at Qwen3-8B 6.6 / 7.0,
+// 100 keys 7.4 / 8.6, 1 x 64 rows of 300 11.4 / 13.4, 1 x 9 rows of 1600 at
+// Qwen3-32B 13.2 / 14.7; past a workgroup a CU the wide tiles win, 4 x 32 rows of
+// 200 keys 15.5 / 12.3.
+bool short_tiles(int32_t num_seqs, int32_t hkv, int32_t n_qtiles, int32_t max_k) {
+  const int64_t tiles = static_cast<int64_t>(num_seqs) * hkv * n_qtiles;
+  const int64_t cus = device_cus();
+  if (max_k <= kMinSplit) return 2 * tiles <= 3 * cus;
+  return tiles * ((max_k + kMinSplit - 1) / kMinSplit) < cus;
+}
+
 size_t partials_bytes(int32_t num_tokens, int32_t hq, int32_t max_splits) {
   const size_t slots = static_cast<size_t>(num_tokens) * hq * max_splits;
   return slots * kD * sizeof(float) + slots * sizeof(float) +
@@ -2085,8 +2110,12 @@ size_t workspace_bytes(int32_t num_seqs, int32_t num_tokens, int32_t hq, int32_t
   const int32_t n_qtiles = (max_q + qtile - 1) / qtile;
   if (n_qtiles > 1) {
     if (group < 1 || group > 64) return 0;   // refused at the launch
-    const WidePlan w = wide_plan(num_seqs, num_tokens, hkv, group, max_q, max_k);
-    return w.max_splits > 1 ? partials_bytes(num_tokens, hq, w.max_splits) : 0;
+    int32_t ms = wide_plan(num_seqs, num_tokens, hkv, group, max_q, max_k).max_splits;
+    if (short_tiles(num_seqs, hkv, n_qtiles, max_k)) {
+      const int32_t tile_ms = (max_k + kMinSplit - 1) / kMinSplit;
+      ms = tile_ms > ms ? tile_ms : ms;
+    }
+    return ms > 1 ? partials_bytes(num_tokens, hq, ms) : 0;
   }
   const int nt = tile_mfmas(qtile * (hkv > 0 ? hq / hkv : 1));
   // either KV dtype: the larger split count of the two wave choices
@@ -2207,13 +2236,15 @@ int run_attention(AttnParams& p, int kv_dtype, void* workspace, size_t workspace
       p.blk_stride % vec_elems || p.tok_stride % vec_elems || p.head_stride % vec_elems)
     return NVA_ERR_UNSUPPORTED;
   const bool fp8 = kv_dtype == NVA_KV_FP8_E4M3;
-  const bool wide = p.n_qtiles > 1;
+  const bool few = p.n_qtiles > 1 && !fp8 && tile_choice().wpt &&
+                   short_tiles(p.num_seqs, p.hkv, p.n_qtiles, p.max_k);
+  const bool wide = p.n_qtiles > 1 && !few;
   const bool stream = stream_mode(p.num_seqs, p.hkv, p.max_q, p.max_k, p.qtile, p.group, fp8);
   const int nt = tile_mfmas(tile_rows);
   // paired mode's whole-sequence split must fit the kernel's block ids
   const int32_t mk = p.max_k > 1 ? p.max_k : 1;
   const int32_t whole = (mk + kMinSplit - 1) / kMinSplit * kMinSplit;
-  const bool paired = !wide && !stream && paired_mode(p.num_seqs, p.hkv, p.max_k, nt, fp8) &&
+  const bool paired = !wide && !few && !stream && paired_mode(p.num_seqs, p.hkv, p.max_k, nt, fp8) &&
                       whole / p.block_size + 2 <= kWave;
   int wps = segment_waves(nt, fp8), key_groups = 1;
   dim3 grid;
@@ -2227,6 +2258,10 @@ int run_attention(AttnParams& p, int kv_dtype, void* workspace, size_t workspace
     p.n_qtiles = w.n_qtiles;
     p.split_len = w.split_len;
     p.max_splits = w.max_splits;
+    grid = dim3(p.hkv, p.num_seqs, p.max_splits * p.n_qtiles);
+  } else if (few) {
+    p.split_len = kMinSplit;
+    p.max_splits = (mk + kMinSplit - 1) / kMinSplit;
     grid = dim3(p.hkv, p.num_seqs, p.max_splits * p.n_qtiles);
   } else if (stream) {
     // a range may span at most kWave - 2 whole blocks (one block id per lane)

@@ -1180,8 +1180,16 @@ WIDE_LARGE = [
                               first=2500)),
     # one sequence of 65 tiles past the 64 page ids
     ("eight_waves_pages", dict(q_len=[257], ctx_lo=2100, ctx_hi=2100, hq=256, hkv=8, block_size=32)),
+    # a few short sequences (bf16: 64-row tiles), unsplit and split, groups that
+    # divide a tile and groups that do not
+    ("64_keys_few", dict(q_len=[30, 17, 64, 0, 1], ctx_lo=64, ctx_hi=64, hq=64, hkv=8, block_size=32)),
+    ("short_few", dict(q_len=[33, 70], ctx_lo=70, ctx_hi=400, hq=16, hkv=8, block_size=32)),
+    ("short_group3", dict(q_len=[50, 22, 0, 64], ctx_lo=1, ctx_hi=260, hq=12, hkv=4, block_size=32)),
+    ("short_group40", dict(q_len=[11, 7, 1], ctx_lo=1, ctx_hi=700, hq=40, hkv=1, block_size=64)),
     # short sequences: one step, two steps, the first past them
-    ("64_keys", dict(q_len=[30, 17, 64, 0, 1], ctx_lo=64, ctx_hi=64, hq=64, hkv=8, block_size=32)),
+    ("64_keys", dict(q_len=[30, 17, 64, 0, 1] * 2, ctx_lo=64, ctx_hi=64, hq=64, hkv=8, block_size=32)),
+    ("group1", dict(q_len=[300, 66, 130], ctx_lo=66, ctx_hi=330, hq=8, hkv=8, block_size=32)),
+    ("group40", dict(q_len=[30, 7, 40, 22], ctx_lo=64, ctx_hi=250, hq=80, hkv=2)),
     ("128_keys", dict(q_len=[30, 17, 90, 128], ctx_lo=128, ctx_hi=128, hq=64, hkv=8, block_size=32)),
     ("129_keys", dict(q_len=[30, 17, 90, 128], ctx_lo=129, ctx_hi=129, hq=64, hkv=8, block_size=32)),
     # splits of 128 keys, four waves and one group
@@ -1298,6 +1306,9 @@ WIDE_CLIPPED = [
     ("two_groups_32_heads", 140, dict(q_len=[150, 141, 139, 0, 160], ctx_lo=150, ctx_hi=400, hq=32,
                                       hkv=8)),
     ("two_groups_64_heads", 70, dict(q_len=[80, 71, 69, 100, 75], ctx_lo=70, ctx_hi=300, hq=64, hkv=8)),
+    # a few short sequences: bf16 on 64-row tiles, unsplit and split
+    ("short_32_heads", 30, dict(q_len=[33, 12, 31], ctx_lo=33, ctx_hi=120, hq=32, hkv=8, block_size=32)),
+    ("short_splits_64_heads", 10, dict(q_len=[11, 0, 17], ctx_lo=300, ctx_hi=380, hq=64, hkv=8)),
     # one or two tiles: two key groups and key splits
     ("splits_16_heads", 40, dict(q_len=[45, 40], ctx_lo=600, ctx_hi=900, hq=16, hkv=8)),
     ("splits_32_heads", 30, dict(q_len=[33, 12, 31], ctx_lo=700, ctx_hi=900, hq=32, hkv=8)),
