@@ -178,9 +178,11 @@ class ModelRunner:
         before serving (model_runner.py:195, :1472-1523): the verify (target
         forward, LM head, fused argmax + accept), the k-step draft, the
         device commit behind the verify and the next step's draft behind
-        both.  Largest bucket first, so the shared attention and argmax
-        workspaces reach their final size before the smaller captures.
-        Buckets a step needs later (a batch above max_num_seqs cannot occur)
+        both.  Largest bucket first: the shared attention and argmax
+        workspaces start at its size.  A smaller bucket, whose sequences are
+        split further, may still need a larger one; each bucket runs eagerly
+        before its capture, and a superseded buffer stays alive for the graphs
+        that hold it.  Buckets a step needs later (a batch above max_num_seqs cannot occur)
         are captured on first use."""
         k = self.speculative_config.num_speculative_tokens
         for bs in reversed(self.eagle3_graph_batch_sizes()):

@@ -225,8 +225,12 @@ int nva_argmax_rows(const void *logits, int64_t row_stride, int32_t vocab, int32
  *   GQA: query head h reads kv head h / (num_q_heads / num_kv_heads).
  *   head_dim must be 128, block_size a multiple of 32 and
  *      num_q_heads / num_kv_heads <= 64; any query length is accepted.
- *   workspace: nva_paged_attention_workspace_size(...) bytes (split-KV
- *      partial results; needs no initialisation).
+ *   workspace: nva_paged_attention_workspace_size(...) bytes for the call's
+ *      own shape, either KV dtype (split-KV partial results; needs no
+ *      initialisation).  Fewer sequences are split further, so the size of a
+ *      larger batch covers a smaller one only where max_seqlen_q *
+ *      num_q_heads / num_kv_heads <= 32 and the larger one has at most 512
+ *      sequences; elsewhere size it for the largest of the shapes' answers.
  * ------------------------------------------------------------------- */
 
 /* Replaces flash_attn_varlen_func(q, k_cache, v_cache, max_seqlen_q,

@@ -146,3 +146,28 @@ def test_attention_workspace_covers_every_layout():
     assert got >= need, (got, need)
     # a bf16-only shape: no split at all needs no workspace beyond zero
     assert lib.nva_paged_attention_workspace_size(64, 384, 32, 8, 128, 6, 1024) >= 0
+
+
+def test_attention_workspace_over_batch_sizes():
+    """Query tiles of at most 32 rows: the size of a batch of up to 512
+    sequences covers every smaller one.  Larger tiles and several tiles are
+    split by how many segments there are: no such promise, the answers are per
+    shape (a larger batch's may be smaller)."""
+    lib = _native.load()
+
+    def sizes(hq, q, max_k):
+        return [lib.nva_paged_attention_workspace_size(b, b * q, hq, 8, 128, q, max_k)
+                for b in range(1, 513)]
+
+    for hq, q in ((16, 1), (16, 5), (32, 1), (32, 6), (32, 8), (64, 1), (64, 4)):
+        for max_k in (1, 128, 129, 1900, 2816, 4096, 16384):
+            got = sizes(hq, q, max_k)
+            assert got == sorted(got), (hq, q, max_k)
+    got = sizes(64, 8, 1900)
+    assert max(got) > got[-1]
+    # every answer covers the partials of the splits it stands for: one slot of
+    # 128 floats and a log-sum-exp per (row, head, split), a count per row
+    slot = 64 * (128 * 4 + 4)
+    for b, n in enumerate(got, 1):
+        rows = 8 * b
+        assert n == 0 or n >= 2 * rows * slot + 4 * rows, b
