@@ -17,14 +17,12 @@
 // has (M 32, N 4096, K 4096: 14.2 us against 11.7).  The waves' sums meet in
 // LDS in wave order (deterministic).
 //
-// Measured on MI355X against the library (rotating weights, us):
-//   N 4096 K 4096:    M 1 9.3 / 15.3   M 16 10.7 / 15.5   M 32 11.7 / 13.6
-//   N 24576 K 4096:   M 1 36.7 / 45.1  M 16 42.2 / 45.3
-//   N 151936 K 4096:  M 1 200 / 250    M 16 225 / 253     M 32 280 / 264
-//   N 4096 K 1024:    M 1 4.4 / 6.5    M 32 4.9 / 8.8     M 64 6.3 / 9.3
-//   N 1024 K 3072:    M 1 6.4 / 9.3    M 32 7.8 / 8.0     M 64 10.8 / 10.5
-//   N 6144 K 8192:    M 1 25.3 / 22.4  M 16 26.7 / 23.8
-//   N 5120 K 25600:   M 1 64 / 134     M 64 106 / 157
+// Measured on MI355X against the library (device time, rotating weights, us):
+//   N 4096 K 4096:    M 1 9.3 / 15.8   M 16 10.1 / 15.8   M 32 11.9 / 13.3
+//   N 24576 K 4096:   M 1 37.0 / 45.4  M 16 42.8 / 45.8
+//   N 4096 K 1024:    M 1 4.0 / 6.1    M 32 4.4 / 8.4     M 64 5.9 / 8.7
+//   N 1024 K 3072:    M 1 6.0 / 9.3    M 32 7.4 / 7.7
+//   N 5120 K 25600:   M 1 68 / 134     M 16 87 / 138      M 64 154 / 157
 #include "common.h"
 
 namespace nva {
@@ -143,20 +141,37 @@ linear_rows_kernel(const uint16_t* __restrict__ x, int64_t x_stride, const uint1
 
 using namespace nva;
 
-// Where the lines lie (us here / library, both sides of each):
+// Where the lines lie (device time, us here / library, rotating weights):
 //   * K > 4096: every workgroup reads x whole, 16 rows of N 6144 K 8192 26.7 /
-//     23.8, N 4096 K 12288 26.7 / 23.4; but where N is small against K the
-//     library leaves most CUs idle (N 5120 K 25600, M 16: 66 / 138);
-//   * M > 16: wide N loses (M 24, N 151936: 267 / 259, N 24576 48.1 / 48.5),
-//     N 6144 K 4096 is level at M 32 (16.1 / 15.9);
-//   * M > 32: N 6144 K 1024 7.4 / 9.4 and N 4096 K 2048 10.1 / 11.4 at M 64,
-//     but N 6144 K 4096 20.2 / 17.8 and N 1024 K 2048 8.5 / 8.2.
+//     23.8, N 4096 K 12288 26.7 / 23.4.  Past K 16384, though, the library's
+//     time jumps where N is small against K (N 512-6144, K 17408-32768: 43-190
+//     us), and this kernel's does not: N 5120 K 25600, M 1 68 / 134, M 32 106 /
+//     146; N 2048 K 20480, M 16 35 / 61.  At K 16384 itself the library splits
+//     K and wins (N 4096, M 16 34.7 / 31.7), below N 512 too few workgroups
+//     stream (N 64 K 49152, M 1 54 / 34), past K 32768 it is mixed (N 1024, M
+//     24 66 / 62), and from 33 rows x costs more: N from 2048, K to 25600 (N
+//     2048 K 25600, M 64 79 / 80; N 5120 K 27648, M 64 164 / 158);
+//   * up to 12 rows, every N (N 16 K 64, M 1 2.1 / 4.2; N 8192 K 4096 level);
+//   * more rows where the last round of workgroups is nearly empty (N between
+//     4096 and 6144): M 16 K 2560 11.4 / 10.7 (N 6144 K 4096 15.7 / 14.7), M 32
+//     K 3072 16.1 / 12.6, K 2048 11.1 / 12.6 still; M 64 K 64 4.1 / 3.9, K 2048
+//     17.2 / 13.2;
+//   * 17-32 rows: N to 4096 (K 4096, M 32 11.9 / 13.3), and to 8192 for K to
+//     2048 (N 6144 K 3072, M 32 14.0 / 13.0), past N 7168, where the library's
+//     time jumps, to 3072 (N 8192, M 32 14.9 / 17.9; K 4096 18.5 / 17.4);
+//     wider N loses (N 9216 K 2560, M 24 20.8 / 15.3);
+//   * 33-64 rows: N 4096 and N 6144-8192 for K to 2048 (N 4096, M 64 10.3 /
+//     12.6; N 6144 12.6 / 13.5; K 4096 21.0 / 18.3); N 1024 K 2048 8.5 / 8.2.
 extern "C" int nva_linear_preferred(int32_t rows, int32_t n, int32_t k) {
   if (rows < 1 || rows > 64 || k < kChunkK || k % kChunkK || n < 16 || n % 4) return 0;
-  if (k >= 4 * static_cast<int64_t>(n) && k >= 16384) return 1;
-  if (rows <= 16) return k <= 4096;
-  if (rows <= 32) return k <= 4096 && n <= 8192;
-  return k <= 2048 && n >= 4096 && n <= 8192;
+  if (k > 4096)
+    return k > 16384 && k <= 32768 && n >= 512 && n <= 6144 && k >= 4 * static_cast<int64_t>(n) &&
+           (rows <= 32 || (n >= 2048 && k <= 25600));
+  const bool part_round = n > 4096 && n < 6144;
+  if (rows <= 12) return 1;
+  if (rows <= 16) return n <= 4096 || n >= 7168 || k <= (part_round ? 2048 : 3584);
+  if (rows <= 32) return n <= 4096 || (n <= 8192 && k <= (n > 7168 ? 3072 : 2048));
+  return n >= 4096 && n <= 8192 && !part_round && k <= 2048;
 }
 
 extern "C" int nva_linear(const void* x, int64_t x_row_stride, const void* w, void* out,

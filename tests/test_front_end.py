@@ -201,6 +201,45 @@ def test_linear_rows_against_64_bits(cuda, m, n, k):
     assert bool(((got.double() - want).abs() <= bound + 1e-30).all())
 
 
+def test_where_the_few_row_kernel_is_preferred():
+    """The lines of nva_linear_preferred, both sides of each."""
+    f = _native.load().nva_linear_preferred
+    yes = [(1, 16, 64), (1, 4096, 4096), (12, 5120, 4096), (16, 4096, 4096), (16, 24576, 4096),
+           (16, 5120, 2048), (16, 6144, 3584), (16, 7168, 4096), (17, 4096, 4096), (32, 1024, 3072),
+           (32, 5120, 2048), (32, 8192, 3072), (33, 4096, 2048), (64, 4096, 1024), (64, 6144, 2048),
+           (64, 8192, 2048), (1, 512, 16448), (32, 5120, 25600), (32, 512, 32768), (64, 5120, 25600),
+           (64, 2048, 20480)]
+    no = [(0, 4096, 4096), (65, 4096, 1024), (-1, 16, 64), (1, 12, 64), (1, 18, 64), (1, 16, 32),
+          (1, 16, 96), (1, 16, 0), (1, 4096, 4160), (16, 4096, 16384), (1, 64, 16448), (1, 508, 20480),
+          (1, 6148, 32768), (1, 5120, 20416), (1, 1024, 32832), (13, 5120, 2112), (13, 6144, 4096),
+          (17, 4100, 2112), (32, 6144, 3072), (32, 8192, 4096), (32, 8196, 64), (33, 1024, 2048),
+          (33, 5120, 1024), (33, 4096, 2112), (64, 8196, 1024), (64, 1024, 20480), (33, 5120, 27648),
+          (64, 1024, 16384)]
+    for m, n, k in yes:
+        assert f(m, n, k) == 1, (m, n, k)
+    for m, n, k in no:
+        assert f(m, n, k) == 0, (m, n, k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(1, 16, 64), (7, 12288, 1024), (16, 6144, 576), (17, 1024, 1600),
+                                   (32, 4096, 4096), (33, 4096, 1024), (2, 512, 17408),
+                                   (33, 1024, 2048), (16, 4096, 8192), (65, 4096, 1024)])
+def test_linear_runs_where_it_is_preferred(cuda, m, n, k):
+    """K.linear is the few-row kernel where nva_linear_preferred says so (its
+    sums have one order, so its bits) and the library's product elsewhere."""
+    g = torch.Generator(device=cuda).manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device=cuda).to(BF16)
+    w = (torch.randn(n, k, generator=g, device=cuda) * 0.05).to(BF16)
+    lib = _native.load()
+    want = torch.nn.functional.linear(x, w)
+    if lib.nva_linear_preferred(m, n, k):
+        want = torch.empty_like(want)
+        _native.check(lib.nva_linear(x.data_ptr(), k, w.data_ptr(), want.data_ptr(), n, m, n, k,
+                                     K._stream()), "linear")
+    assert torch.equal(K.linear(x, w), want)
+
+
 @pytest.mark.gpu
 def test_linear_takes_every_form_the_library_takes(cuda):
     import torch.nn.functional as F
