@@ -82,7 +82,7 @@ class _Staging:
 
     def __init__(self, sizes: dict[str, int], dtype: torch.dtype, device: torch.device):
         total = sum(sizes.values())
-        self.host = torch.zeros(max(total, 1), dtype=dtype, pin_memory=True)
+        self.host = torch.zeros(max(total, 1), dtype=dtype, device="cpu", pin_memory=True)
         # fields are written through a numpy view of the pinned buffer: a
         # torch tensor built from a list plus a copy_ per field cost the
         # host ~30 us each, on the path between two verify graphs

@@ -20,6 +20,8 @@ token.)
 """
 from __future__ import annotations
 
+from contextlib import contextmanager
+
 import numpy as np
 import torch
 
@@ -51,11 +53,23 @@ def _use_gemm_tuning(path: str) -> None:
 
 
 def _pinned(values, dtype) -> torch.Tensor:
+    """A pinned host copy (host tensors name their device: the caller may have
+    set a default one)."""
     if isinstance(values, np.ndarray):
-        out = torch.empty(values.shape, dtype=dtype, pin_memory=True)
+        out = torch.empty(values.shape, dtype=dtype, device="cpu", pin_memory=True)
         out.copy_(torch.from_numpy(values))
         return out
-    return torch.tensor(values, dtype=dtype, pin_memory=True)
+    return torch.tensor(values, dtype=dtype, device="cpu", pin_memory=True)
+
+
+@contextmanager
+def _default_dtype(dtype):
+    before = torch.get_default_dtype()
+    torch.set_default_dtype(dtype)
+    try:
+        yield
+    finally:
+        torch.set_default_dtype(before)
 
 
 class ModelRunner:
@@ -75,14 +89,14 @@ class ModelRunner:
             _use_gemm_tuning(config.gemm_tuning_file)
         self._exited = False
         self.decode_graph_replay_count = 0
-        default_dtype = torch.get_default_dtype()
         dtype = getattr(hf, "torch_dtype", None) or getattr(hf, "dtype", None) or torch.bfloat16
         if isinstance(dtype, str):
             dtype = getattr(torch, dtype)
         self.dtype = dtype
-        torch.set_default_dtype(dtype)
-        torch.set_default_device(self.device)
-        try:
+        # contexts, so that the caller's own default device (or none: a default
+        # that is set, whichever, sends every torch call through a Python mode)
+        # and dtype are in place again afterwards
+        with _default_dtype(dtype), torch.device(self.device):
             self.model = Qwen3ForCausalLM(hf)
             if config.load_format == "dummy":
                 init_random_(self.model, config.seed)
@@ -128,11 +142,6 @@ class ModelRunner:
                 self.state_feedback = torch.zeros(rows + 1, h, dtype=self.dtype, device=self.device)
                 self._state_slot: dict[int, int] = {}
                 self._free_state = list(range(rows - 1, -1, -1))
-        finally:
-            # not "cpu": a default device that is set, whichever, sends every
-            # later torch call through a Python mode
-            torch.set_default_device(None)
-            torch.set_default_dtype(default_dtype)
         # benchmarks may ask to keep the last verify's logits and inputs, or to
         # run the verify forward eagerly (kernel-level timing)
         self.keep_verify_inputs = False
@@ -156,9 +165,9 @@ class ModelRunner:
         # pipelined steps, and those among them with a sequence proposing
         # fewer than k drafts (close to its budget)
         self.pipeline_stats = {"steps": 0, "ragged": 0}
-        self._proposal_host = torch.empty(0, dtype=torch.int64)
+        self._proposal_host = torch.empty(0, dtype=torch.int64, device="cpu")
         # one pinned host buffer receives argmax + accept results each verify
-        self._verify_host = torch.empty(1 << 16, dtype=torch.int32, pin_memory=True)
+        self._verify_host = torch.empty(1 << 16, dtype=torch.int32, device="cpu", pin_memory=True)
         self._verify_dev = torch.empty(1 << 16, dtype=torch.int32, device=self.device)
         if self.eagle3_model is not None and self._use_graphs():
             self.capture_eagle3_graphs()
@@ -726,7 +735,8 @@ class ModelRunner:
                 by_col[c] = seqs[i]
             self.draft_override(by_col, tokens)
         if self._proposal_host.numel() < k * bs:
-            self._proposal_host = torch.empty(k * bs, dtype=torch.int64, pin_memory=True)
+            self._proposal_host = torch.empty(k * bs, dtype=torch.int64, device="cpu",
+                                              pin_memory=True)
         host = self._proposal_host[:k * bs]
         host.copy_(tokens.reshape(-1), non_blocking=True)
         proposed = torch.cuda.Event()
@@ -850,7 +860,8 @@ class ModelRunner:
                 n = t + 2 * b
                 if n > self._verify_dev.numel():
                     self._verify_dev = torch.empty(2 * n, dtype=torch.int32, device=self.device)
-                    self._verify_host = torch.empty(2 * n, dtype=torch.int32, pin_memory=True)
+                    self._verify_host = torch.empty(2 * n, dtype=torch.int32, device="cpu",
+                                                    pin_memory=True)
                 K.argmax_accept(logits, ctx.cu_seqlens_q, input_ids, out=self._verify_dev[:n])
                 self._verify_host[:n].copy_(self._verify_dev[:n], non_blocking=True)
                 torch.cuda.current_stream().synchronize()

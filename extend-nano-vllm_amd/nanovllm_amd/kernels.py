@@ -382,7 +382,7 @@ def _device_lengths(t, device: torch.device, name: str):
         if t.device != device:
             raise ValueError("all tensors must be on the same device")
         return t, None
-    host = torch.as_tensor(t, dtype=torch.int32)
+    host = torch.as_tensor(t, dtype=torch.int32, device="cpu")
     if host.dim() != 1:
         raise ValueError(f"{name} must be one-dimensional")
     if torch.cuda.is_current_stream_capturing():

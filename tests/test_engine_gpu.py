@@ -550,3 +550,24 @@ def test_prelaunched_drafts_with_the_device_running_behind(dirs, monkeypatch):
         assert a.keys() == b.keys(), step
         for key in a:
             assert torch.equal(a[key], b[key]), step
+
+
+def test_engine_under_the_callers_default_device(dirs):
+    """A default device the caller has set stays set, and the engine's tokens do
+    not depend on it (its host buffers stay on the host)."""
+    ps, sp = prompts(5, seed=9), SamplingParams(temperature=0.0, max_tokens=12, ignore_eos=True)
+    llm = make_llm(dirs)
+    want = [o["token_ids"] for o in llm.generate(ps, sp, use_tqdm=False)]
+    llm.exit()
+    torch.set_default_device("cuda")
+    try:
+        for eager in (True, False):
+            llm = make_llm(dirs, eager=eager)
+            assert torch.get_default_device().type == "cuda"
+            got = [o["token_ids"] for o in llm.generate(ps, sp, use_tqdm=False)]
+            llm.exit()
+            if eager:
+                assert got == want
+            assert [len(t) for t in got] == [12] * 5
+    finally:
+        torch.set_default_device(None)

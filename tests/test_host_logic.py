@@ -576,3 +576,45 @@ def test_draft_steps_past_the_last_proposal_see_written_keys_only():
     assert ctx[:, 0].tolist() == [99, 99, 99, 99] and set(slots[:, 0].tolist()) == {-1}
     assert ctx[:, 1].tolist() == [255, 256, 256, 256] and slots[2:, 1].tolist() == [-1, -1]
     assert ctx[:, 2].tolist() == [40, 41, 42, 43] and min(slots[:, 2].tolist()) >= 0
+
+
+@pytest.mark.parametrize("before", [None, "cpu", "meta"])
+def test_building_an_engine_leaves_the_default_device_and_dtype_alone(monkeypatch, before):
+    """The model is built under the engine's device and dtype; afterwards, also
+    after a failure, the caller's own are in place, or none."""
+    seen = []
+
+    def build(hf):
+        seen.append((torch.get_default_device(), torch.get_default_dtype()))
+        raise RuntimeError("stop here")
+
+    monkeypatch.setattr(mr._native, "load_front_end", lambda: None)
+    monkeypatch.setattr(torch.cuda, "set_device", lambda device: None)
+    monkeypatch.setattr(mr, "Qwen3ForCausalLM", build)
+    config = SimpleNamespace(hf_config=SimpleNamespace(torch_dtype=torch.bfloat16), kvcache_block_size=256,
+                             enforce_eager=True, device_offset=0, gemm_tuning_file=None)
+    modes = torch._C._len_torch_function_stack()
+    torch.set_default_device(before)
+    try:
+        with_own = torch._C._len_torch_function_stack()
+        with pytest.raises(RuntimeError, match="stop here"):
+            mr.ModelRunner(config)
+        assert seen == [(torch.device("cuda", 0), torch.bfloat16)]
+        assert torch.get_default_device() == torch.device(before or "cpu")
+        assert torch._C._len_torch_function_stack() == with_own   # no mode left, none taken away
+        assert torch.get_default_dtype() == torch.float32
+    finally:
+        torch.set_default_device(None)
+    assert torch._C._len_torch_function_stack() == modes
+
+
+def test_host_lengths_stay_on_the_host_under_a_default_device(monkeypatch):
+    from nanovllm_amd import kernels as K
+
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    torch.set_default_device("meta")
+    try:
+        _, host = K._device_lengths([3, 5], torch.device("meta"), "lengths")
+    finally:
+        torch.set_default_device(None)
+    assert host == [3, 5]
