@@ -530,5 +530,12 @@ extern "C" __attribute__((visibility("default"))) PyObject* PyInit__front_end() 
       reinterpret_cast<PyTypeObject*>(PyObject_GetAttrString(device_module, "DeviceContext"));
   Py_DECREF(device_module);
   if (!g_device_context) return nullptr;
-  return PyModule_Create(&module);
+  PyObject* m = PyModule_Create(&module);
+  // what it was built against: the interpreter and torch whose ABI it uses
+  if (m && (PyModule_AddIntConstant(m, "built_for_python", PY_VERSION_HEX >> 16) < 0 ||
+            PyModule_AddStringConstant(m, "built_for_torch", NVA_TORCH_VERSION) < 0)) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
 }

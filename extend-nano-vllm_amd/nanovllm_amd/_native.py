@@ -12,6 +12,7 @@ import importlib.machinery
 import importlib.util
 import os
 import subprocess
+import sys
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG, "lib", "libnanovllm_amd.so")
@@ -90,8 +91,9 @@ _lib: ctypes.CDLL | None = None
 
 
 def build(verbose: bool = False) -> str:
-    """Compile libnanovllm_amd.so for gfx950 with the committed Makefile."""
-    cmd = ["make", "-C", CSRC_DIR, "-j8"]
+    """Compile libnanovllm_amd.so for gfx950, and the front end for this Python
+    and its torch, with the committed Makefile."""
+    cmd = ["make", "-C", CSRC_DIR, "-j8", f"PYTHON={sys.executable}"]
     if not verbose:
         cmd.insert(1, "-s")
     subprocess.run(cmd, check=True)
@@ -125,7 +127,7 @@ def load_front_end():
     """The CPython module in front of the library (csrc/front_end.cpp)."""
     global _front
     if _front is None:
-        import torch  # noqa: F401  - the module links against torch's libraries
+        import torch  # the module links against torch's libraries
         load()
         if not os.path.exists(FRONT_PATH):
             raise NativeLibraryError(f"{FRONT_PATH} is missing: build it with `make -C {CSRC_DIR}` "
@@ -137,6 +139,12 @@ def load_front_end():
             loader.exec_module(module)
         except ImportError as exc:
             raise NativeLibraryError(f"cannot load {FRONT_PATH}: {exc}") from exc
+        built = (module.built_for_python, module.built_for_torch)
+        here = (sys.hexversion >> 16, str(torch.__version__))
+        if built != here:
+            raise NativeLibraryError(f"{FRONT_PATH} was built for Python {built[0]:#x} and torch "
+                                     f"{built[1]}, this is {here[0]:#x} and {here[1]}: build it again "
+                                     f"(`make -C {CSRC_DIR} PYTHON={sys.executable}`)")
         _front = module
     return _front
 

@@ -304,3 +304,30 @@ def test_loads_in_a_process_that_has_not_imported_torch():
     pkg = os.path.dirname(os.path.dirname(os.path.abspath(_native.__file__)))
     subprocess.run([sys.executable, "-c", code], check=True, timeout=300,
                    env={**os.environ, "PYTHONPATH": pkg})
+
+
+def test_a_module_of_another_torch_or_python_is_refused(monkeypatch):
+    """Its ABI is the interpreter's and torch's it was built against."""
+    _native.load_front_end()
+    monkeypatch.setattr(_native, "_front", None)
+    with monkeypatch.context() as m:
+        m.setattr(torch, "__version__", "0.0.1")
+        with pytest.raises(_native.NativeLibraryError, match="0.0.1.*build it again"):
+            _native.load_front_end()
+    with monkeypatch.context() as m:
+        m.setattr(_native.sys, "hexversion", 0x03000000)
+        with pytest.raises(_native.NativeLibraryError, match="0x300.*build it again"):
+            _native.load_front_end()
+    assert _native.load_front_end().built_for_torch == torch.__version__
+
+
+def test_the_front_end_is_built_again_when_torch_changes(tmp_path):
+    """make would run the module's rule for another interpreter's torch."""
+    fake = tmp_path / "torch"
+    fake.mkdir()
+    (fake / "__init__.py").write_text("")
+    (fake / "version.py").write_text("__version__ = '9.9.9'\n")
+    out = subprocess.run(["make", "-n", "-C", _native.CSRC_DIR, f"PYTHON={sys.executable}"],
+                         env={**os.environ, "PYTHONPATH": str(tmp_path)}, capture_output=True, text=True,
+                         check=True, timeout=120).stdout
+    assert "9.9.9" in out and f"-I{fake}" not in out and f"{fake}/include" in out
