@@ -588,7 +588,7 @@ def add_rms_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, 
 def merge_heads(x: torch.Tensor) -> torch.Tensor:
     """[T, H, D] as [T, H * D]."""
     got = (_front or _front_end()).merge_heads(x)
-    return x.reshape(x.shape[0], -1) if got is None else got
+    return x.flatten(1) if got is None else got
 
 
 def place(x: torch.Tensor) -> tuple:

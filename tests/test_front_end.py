@@ -49,6 +49,7 @@ def test_refusals_are_the_python_paths():
         K.paged_attention_varlen(x, x, x, x, x, 1, 1, 1.0, x, causal=False)
     assert K.place(x) == (None, 16)
     assert K.merge_heads(torch.zeros(2, 3, 4)).shape == (2, 12)
+    assert K.merge_heads(torch.zeros(0, 3, 4)).shape == (0, 12)
 
 
 def _both(monkeypatch, call):
