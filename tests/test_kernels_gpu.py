@@ -754,6 +754,39 @@ def test_qk_norm_rope_store_matches_separate_kernels(K, cuda, layout, fp8, with_
     assert changed.any()
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hq,hkv", [(4, 1), (5, 1), (6, 2), (5, 3), (7, 7), (12, 2), (13, 4), (16, 5)])
+def test_qk_norm_rope_head_counts(K, cuda, hq, hkv, fp8):
+    """Head counts around the fours that a wave takes: each kind of head where
+    it belongs, every one equal to the same head alone (one query, one kv head
+    a launch, whose values the tests above hold to the formulas)."""
+    d, nb, bs, t = 128, 2, 32, 40
+    g, qkv, pos, qw, kw, cos_sin = _layer_case(35, t=t, hq=hq, hkv=hkv)
+    slots = torch.randperm(nb * bs, generator=g)[:t].to(torch.int32)
+    cdt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    init = torch.randn(nb, bs, hkv, d, generator=g).to(cdt)
+    kc, vc = init.clone().to(cuda), init.clone().to(cuda)
+    dq, dpos, dslots, dqw, dkw = (x.to(cuda) for x in (qkv, pos, slots, qw, kw))
+    q, k = K.qk_norm_rope(dq, dpos, dqw, dkw, cos_sin, hq, hkv, d, 1e-6)
+    q2 = K.qk_norm_rope_store(dq, dpos, dqw, dkw, cos_sin, hq, hkv, d, 1e-6, kc, vc, dslots)
+    assert torch.equal(q, q2)
+    heads = dq.view(t, hq + 2 * hkv, d)
+    for i in range(max(hq, hkv)):
+        j = min(i, hkv - 1)
+        one = torch.stack([heads[:, min(i, hq - 1)], heads[:, hq + j], heads[:, hq + hkv + j]], 1)
+        kc1, vc1 = (init[:, :, j:j + 1].clone().to(cuda) for _ in range(2))
+        q1 = K.qk_norm_rope_store(one.reshape(t, 3 * d), dpos, dqw, dkw, cos_sin, 1, 1, d, 1e-6, kc1,
+                                  vc1, dslots)
+        assert torch.equal(q[:, min(i, hq - 1)], q1[:, 0]), i
+        np.testing.assert_array_equal(bits(kc[:, :, j].cpu()), bits(kc1[:, :, 0].cpu()))
+        np.testing.assert_array_equal(bits(vc[:, :, j].cpu()), bits(vc1[:, :, 0].cpu()))
+    kb = torch.zeros_like(kc)
+    K.store_kvcache(k, heads[:, hq + hkv:].contiguous(), kb, torch.zeros_like(vc), dslots)
+    written = dslots.cpu().long()
+    np.testing.assert_array_equal(bits(kc.cpu().view(nb * bs, hkv, d)[written]),
+                                  bits(kb.cpu().view(nb * bs, hkv, d)[written]))
+
+
 @pytest.mark.parametrize("inter", [1000, 4104])
 def test_silu_mul_vector_path_matches_scalar_and_reference(K, cuda, inter):
     """16-byte vector path == element path (bit-exact); both within one bf16
