@@ -189,9 +189,10 @@ rms_norm_kernel(const uint16_t* __restrict__ x, int64_t x_stride,
 //
 // Memory bound at prefill sizes, latency bound below.  16 lanes take a head:
 // lane i the elements 4 i .. 4 i + 3 and 64 + 4 i .. (the two halves the
-// rotation pairs) as 8-byte loads and stores, four heads a wave.  With a head
-// a wave and 2-byte accesses, 384 tokens of 48 heads took 7.7 us, 1024 of 32
-// heads 12.2, 16384 of 48 heads 177 (2.3 TB/s); now 5.1, 6.0 and 72.6 (5.5).
+// rotation pairs) as 8-byte loads and stores, four heads a wave.  Against a head
+// a wave with 2-byte accesses, us (20 launches in a graph): 384 tokens of 48
+// heads 6.6 -> 4.4, 1024 of 32 heads 10.7 -> 4.7, 16384 of 48 heads 174 (2.3
+// TB/s) -> 65.6 (6.1); FP8 pages 7.5 -> 5.0, 13.5 -> 6.4, 194 -> 74.
 enum class KeyTo { kTensor, kCacheBf16, kCacheFp8 };
 
 struct SlotPages {

@@ -832,8 +832,9 @@ __device__ __forceinline__ int stream_chunks(const AttnParams& p, int seq) {
 }
 
 // Fixed decomposition, WPS waves per (kv head, sequence, split).
-// Dispatch order (x fastest): kv head, sequence, then the split slowest, so every full split is dispatched before the shorter trailing
-// splits and the empty splits that pad the grid come last.
+// Dispatch order (x fastest): kv head, sequence, then the split slowest, so
+// every full split is dispatched before the shorter trailing splits and the
+// empty splits that pad the grid come last.
 // Two waves per SIMD fit the register budget of tiles up to 32 columns;
 // 64-column tiles (NT = 4) need the full register file of one wave.
 template <int NT, bool FP8, bool PIPE, int WPS>
@@ -1206,13 +1207,14 @@ paged_attention_tile_kernel(AttnParams p) {
 //     first's through LDS at the end (wide_plan says when).
 // Against the 64-row tiles (which read K and V from LDS once per 16 columns
 // and from L2 once per 64 rows; FP8 ones on one wave): 16384 tokens as
-// 8192-token prompts at Qwen3-8B 2974 -> 1091 us (370 -> 1008 TFLOP/s of the
-// unmasked products; MFMAs busy 47% of the cycles), 256-2048-token prompts
-// 511 -> 314, over FP8 pages 4196 -> 1045 and 536 -> 256.  What was tried and
-// did not help: the next step's scores issued among this step's exponentials
-// (spills: 1389 us), s_setprio around the MFMAs (1117), query and output rows
-// through LDS as whole lines (+0-4%), light and heavy query tiles alternated
-// (+5%).
+// 8192-token prompts at Qwen3-8B 2957 -> 1116 us (372 -> 985 TFLOP/s of the
+// unmasked products; MFMAs busy 45% of the cycles), 256-2048-token prompts
+// 534 -> 308 (27%: part tiles, and the start of short sequences), over FP8
+// pages 4152 -> 1075 and 529 -> 244.  What was tried and did not help (on a box
+// where the first took 1091): the next step's scores issued among this step's
+// exponentials (spills: 1389 us), s_setprio around the MFMAs (1117), query and
+// output rows through LDS as whole lines (+0-4%), light and heavy query tiles
+// alternated (+5%).
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 constexpr int kWideKeys = 64;
 constexpr int kWideKPitch = 68, kWideVPitch = 80;   // dwords per staged row
@@ -1808,6 +1810,9 @@ TileChoice tile_choice() {
 //     1024 keys, where a share is short, one more pays when lengths spread
 //     (400 of 600 r 2 42.7 / 37.1), also halves of 1024-3328 keys (640 of 3200
 //     r 4 151 / 124, r 1 160 / 218, whole 212); nine shares or more hide it.
+//     Elsewhere spread lengths give up what a share more would win them (456
+//     of 1036-3761 keys 135 / 98; up to 1.2x at most shapes), equal ones keep
+//     up to 1.6x.
 //   * single waves of up to 32 rows share a SIMD two by two: one share more.
 // Against the rule of at least 1024 waves that shrank the default length
 // before, alternating on one box, us: Qwen3-0.6B decode 4 x 4000-8000 keys 33.9
